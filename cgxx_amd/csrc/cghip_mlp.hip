@@ -1,8 +1,8 @@
 // C ABI of the FP32 network (declared in include/cghip_mlp.h).
 //
 // The handle owns one stream and the device buffers: parameters, Adam
-// moments, the inputs/targets of up to max_rows rows, the activations, the
-// partial gradients of the backward blocks and the per-step losses.
+// moments, the inputs/targets of up to max_rows rows, the activations and
+// deltas of every layer and the per-step losses.
 
 #include "../../include/cghip_mlp.h"
 #include "mlp.h"
@@ -17,8 +17,6 @@
 using namespace cghip;
 
 namespace {
-
-constexpr int kBackwardBlocks = 128;  // partial-gradient slices
 
 bool valid_dims(int in, int h1, int h2, int out) {
   auto ok = [](int w) { return w >= 1 && w <= kMlpMaxWidth; };
@@ -36,7 +34,8 @@ struct cghip_mlp {
   MlpDims d{};
   int total = 0, max_rows = 0, step = 0;
   float *P = nullptr, *M = nullptr, *V = nullptr, *grad = nullptr;
-  float *X = nullptr, *T = nullptr, *A1 = nullptr, *A2 = nullptr, *Y = nullptr, *Gp = nullptr;
+  float *X = nullptr, *T = nullptr, *Y = nullptr;
+  MlpTables tab{};
   double *Lp = nullptr, *loss = nullptr;
   int loss_cap = 0;
 };
@@ -87,11 +86,11 @@ int sync(cghip_mlp *m) {
   return 0;
 }
 
-// Forward with activations kept, then the backward pass into Gp / Lp.
-int forward_backward(cghip_mlp *m, int rows, int G) {
-  MLPCHK(m, mlp_forward(m->d, m->P, m->X, rows, m->A1, m->A2, m->Y, m->stream));
-  MLPCHK(m, mlp_backward(m->d, m->P, m->X, m->A1, m->A2, m->Y, m->T, rows, G, m->Gp, m->Lp,
-                         m->stream));
+// Forward, backward, then the gradient (into `grad` when non-null) with the
+// Adam step `a` and the loss.
+int train_step(cghip_mlp *m, int rows, float *grad, const AdamStep &a, double *loss) {
+  MLPCHK(m, mlp_backprop(m->d, m->P, m->X, m->T, rows, m->tab, m->Lp, m->stream));
+  MLPCHK(m, mlp_gradient(m->d, rows, m->tab, grad, m->P, m->M, m->V, a, m->Lp, loss, m->stream));
   return 0;
 }
 
@@ -120,7 +119,9 @@ int cghip_mlp_destroy(cghip_mlp *m) {
   (void)hipSetDevice(m->device);
   if (m->stream) (void)hipStreamSynchronize(m->stream);
   release(m->P), release(m->M), release(m->V), release(m->grad);
-  release(m->X), release(m->T), release(m->A1), release(m->A2), release(m->Y), release(m->Gp);
+  release(m->X), release(m->T), release(m->Y);
+  for (float *&p : m->tab.in) release(p);
+  for (float *&p : m->tab.delta) release(p);
   release(m->Lp), release(m->loss);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
@@ -155,11 +156,16 @@ int cghip_mlp_create(int device, int in, int h1, int h2, int out, int max_rows, 
   if (!rc) rc = alloc(m, &m->grad, P);
   if (!rc) rc = alloc(m, &m->X, R * in);
   if (!rc) rc = alloc(m, &m->T, R * out);
-  if (!rc) rc = alloc(m, &m->A1, R * h1);
-  if (!rc) rc = alloc(m, &m->A2, R * h2);
   if (!rc) rc = alloc(m, &m->Y, R * out);
-  if (!rc) rc = alloc(m, &m->Gp, (size_t)kBackwardBlocks * P);
-  if (!rc) rc = alloc(m, &m->Lp, kBackwardBlocks);
+  if (!rc) rc = alloc(m, &m->tab.in[0], R * (in + 1));
+  if (!rc) rc = alloc(m, &m->tab.in[1], R * (h1 + 1));
+  if (!rc) rc = alloc(m, &m->tab.in[2], R * (h2 + 1));
+  if (!rc) rc = alloc(m, &m->tab.delta[0], R * h1);
+  if (!rc) rc = alloc(m, &m->tab.delta[1], R * h2);
+  if (!rc) rc = alloc(m, &m->tab.delta[2], R * out);
+  if (!rc) rc = alloc(m, &m->Lp, (R + 3) / 4);
+  if (!rc && (e = mlp_prepare()) != hipSuccess)
+    rc = fail(m, 2, "mlp_prepare: %s", hipGetErrorString(e));
   if (!rc && (e = hipMemsetAsync(m->P, 0, sizeof(float) * P, m->stream)) != hipSuccess)
     rc = fail(m, 2, "hipMemset: %s", hipGetErrorString(e));
   if (!rc && (e = hipMemsetAsync(m->M, 0, sizeof(float) * P, m->stream)) != hipSuccess)
@@ -203,7 +209,7 @@ int cghip_mlp_forward(cghip_mlp *m, const float *X, int rows, float *Y) {
   if (int rc = check_rows(m, rows)) return rc;
   MLPCHK(m, hipSetDevice(m->device));
   if (int rc = upload_rows(m, X, nullptr, rows)) return rc;
-  MLPCHK(m, mlp_forward(m->d, m->P, m->X, rows, nullptr, nullptr, m->Y, m->stream));
+  MLPCHK(m, mlp_forward(m->d, m->P, m->X, rows, m->Y, m->stream));
   MLPCHK(m, hipMemcpyAsync(Y, m->Y, sizeof(float) * (size_t)rows * m->d.out, hipMemcpyDeviceToHost,
                            m->stream));
   return sync(m);
@@ -216,18 +222,15 @@ int cghip_mlp_gradient(cghip_mlp *m, const float *X, const float *T, int rows, f
   if (int rc = check_rows(m, rows)) return rc;
   MLPCHK(m, hipSetDevice(m->device));
   if (int rc = upload_rows(m, X, T, rows)) return rc;
-  const int G = std::min(rows, kBackwardBlocks);
-  if (int rc = forward_backward(m, rows, G)) return rc;
-  AdamStep a{};
-  a.apply = 0;
-  MLPCHK(m, mlp_adam(m->total, G, m->Gp, m->grad, m->P, m->M, m->V, a, m->stream));
   if (m->loss_cap < 1) {
     release(m->loss);
     m->loss_cap = 0;
     if (int rc = alloc(m, &m->loss, 1)) return rc;
     m->loss_cap = 1;
   }
-  MLPCHK(m, mlp_loss(G, m->Lp, (double)rows * m->d.out, m->loss, m->stream));
+  AdamStep a{};
+  a.apply = 0;
+  if (int rc = train_step(m, rows, m->grad, a, m->loss)) return rc;
   MLPCHK(m, hipMemcpyAsync(grad, m->grad, sizeof(float) * m->total, hipMemcpyDeviceToHost, m->stream));
   MLPCHK(m, hipMemcpyAsync(loss, m->loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
   return sync(m);
@@ -250,10 +253,7 @@ int cghip_mlp_train(cghip_mlp *m, const float *X, const float *T, int rows, int 
     if (int rc = alloc(m, &m->loss, (size_t)std::max(steps, 1))) return rc;
     m->loss_cap = std::max(steps, 1);
   }
-  const int G = std::min(rows, kBackwardBlocks);
   for (int s = 0; s < steps; s++) {
-    if (int rc = forward_backward(m, rows, G)) return rc;
-    MLPCHK(m, mlp_loss(G, m->Lp, (double)rows * m->d.out, m->loss + s, m->stream));
     const int t = ++m->step;
     AdamStep a;
     a.lr = o->lr;
@@ -263,7 +263,7 @@ int cghip_mlp_train(cghip_mlp *m, const float *X, const float *T, int rows, int 
     a.corr1 = (float)(1.0 / (1.0 - std::pow((double)o->beta1, t)));
     a.corr2 = (float)(1.0 / (1.0 - std::pow((double)o->beta2, t)));
     a.apply = 1;
-    MLPCHK(m, mlp_adam(m->total, G, m->Gp, nullptr, m->P, m->M, m->V, a, m->stream));
+    if (int rc = train_step(m, rows, nullptr, a, m->loss + s)) return rc;
   }
   if (loss_history && steps > 0)
     MLPCHK(m, hipMemcpyAsync(loss_history, m->loss, sizeof(double) * steps, hipMemcpyDeviceToHost,

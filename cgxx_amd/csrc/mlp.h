@@ -19,17 +19,36 @@ struct AdamStep {
 
 int mlp_param_count(const MlpDims &d);
 
-// A1/A2 (rows x h1 / h2, nullable) keep the activations for the backward pass.
-hipError_t mlp_forward(const MlpDims &d, const float *P, const float *X, int rows, float *A1,
-                       float *A2, float *Y, hipStream_t s);
-// Partial gradients Gp[G][total] and loss shares Lp[G] of the MSE loss.
-hipError_t mlp_backward(const MlpDims &d, const float *P, const float *X, const float *A1,
-                        const float *A2, const float *Y, const float *T, int rows, int G, float *Gp,
-                        double *Lp, hipStream_t s);
-// Folds Gp into the gradient (copied to `grad` when non-null) and, when
-// a.apply, takes one Adam step on P with moments M, V.
-hipError_t mlp_adam(int total, int G, const float *Gp, float *grad, float *P, float *M, float *V,
-                    const AdamStep &a, hipStream_t s);
-hipError_t mlp_loss(int G, const double *Lp, double denom, double *out, hipStream_t s);
+// Blocks (and loss shares) of mlp_backprop for `rows` samples.
+int mlp_tiles(int rows);
+
+// Of every layer k what mlp_backprop leaves for mlp_gradient, one row per
+// sample: its inputs followed by a 1 (in[k], widths in + 1, h1 + 1, h2 + 1)
+// and its deltas (delta[k], widths h1, h2, out).
+struct MlpTables {
+  float *in[3], *delta[3];
+};
+
+// Slices of the samples whose gradient sums are formed apart (slice g:
+// samples g, g + G, ...; G = min(rows, kMlpSlices)), and the table rows of
+// one lane in the gradient kernel: a block keeps kMlpSlices * kMlpGradRows *
+// 64 slice sums, 64 KB, in LDS.
+constexpr int kMlpSlices = 128;
+constexpr int kMlpGradRows = 2;
+
+// Once per device before mlp_backprop.
+hipError_t mlp_prepare();
+
+hipError_t mlp_forward(const MlpDims &d, const float *P, const float *X, int rows, float *Y,
+                       hipStream_t s);
+// Forward and backward of the MSE loss: the tables and the loss shares
+// Lp[mlp_tiles(rows)].
+hipError_t mlp_backprop(const MlpDims &d, const float *P, const float *X, const float *T, int rows,
+                        const MlpTables &tab, double *Lp, hipStream_t s);
+// The gradient (copied to `grad` when non-null), when a.apply one Adam step
+// on P with moments M, V, and the loss.
+hipError_t mlp_gradient(const MlpDims &d, int rows, const MlpTables &tab, float *grad, float *P,
+                        float *M, float *V, const AdamStep &a, const double *Lp, double *loss,
+                        hipStream_t s);
 
 }  // namespace cghip
