@@ -43,6 +43,10 @@ struct cghip_ctx {
   int *ell_length = nullptr, *ell_index = nullptr;
   double *ell_data = nullptr;
 
+  // the symmetric diagonals of each, where the matrix has them (pairs > 0):
+  // read instead of the arrays by every FP64 product
+  Sym64 crs_sym{}, ell_sym{};
+
   bool has_jac = false;
   double *jac = nullptr;
 
@@ -197,7 +201,14 @@ void free_fp32(cghip_ctx *c) {
   c->poly_degree = 0;
 }
 
+void free_sym(Sym64 &s) {
+  if (s.diag) (void)hipFree((void *)s.diag);
+  if (s.up) (void)hipFree((void *)s.up);
+  s = Sym64{};
+}
+
 void free_crs(cghip_ctx *c) {
+  free_sym(c->crs_sym);
   dfree(c->crs_ptr);
   dfree(c->crs_index);
   dfree(c->crs_value);
@@ -207,6 +218,7 @@ void free_crs(cghip_ctx *c) {
 }
 
 void free_ell(cghip_ctx *c) {
+  free_sym(c->ell_sym);
   dfree(c->ell_length);
   dfree(c->ell_index);
   dfree(c->ell_data);
@@ -289,13 +301,86 @@ int check_ready(cghip_ctx *c) {
   return CGHIP_OK;
 }
 
+int sync(cghip_ctx *c) {
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return CGHIP_OK;
+}
+
+const Sym64 &sym_of(const cghip_ctx *c) {
+  return c->format == CGHIP_FORMAT_CRS ? c->crs_sym : c->ell_sym;
+}
+
+// Bytes per row that one FP64 product reads of the matrix.
+int64_t matrix_row_bytes(const cghip_ctx *c) {
+  if (sym_of(c).pairs) return 8 * (1 + sym_of(c).pairs);
+  return 4 + (c->format == CGHIP_FORMAT_CRS ? 12 * (int64_t)c->crs_nnz / c->n
+                                            : 12 * (int64_t)c->ell_width);
+}
+
 hipError_t launch_matvec(cghip_ctx *c, const double *x, double *y) {
+  if (sym_of(c).pairs) return matvec_sym64(sym_of(c), x, y, c->stream);
   if (c->format == CGHIP_FORMAT_CRS) return matvec_crs(crs_of(c), x, y, c->stream);
   return matvec_ell(ell_of(c), x, y, c->stream);
 }
 
-int sync(cghip_ctx *c) {
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+// Distinct off-diagonal offsets j - i of an uploaded matrix, ascending.
+struct Offsets {
+  int count = -1;  // -1: more than kDiaMax, or columns out of order
+  int off[kDiaMax] = {};
+  bool marked = false;  // an entry is kF64Absent
+};
+
+template <typename M>
+int find_offsets(cghip_ctx *c, const M &A, Offsets *out) {
+  int *found = reinterpret_cast<int *>(c->partial);
+  int h[kDiaMax + 1];
+  HIPCHK(c, matrix_offsets(A, found, c->stream));
+  HIPCHK(c, hipMemcpyAsync(h, found, sizeof(h), hipMemcpyDeviceToHost, c->stream));
+  if (int rc = sync(c)) return rc;
+  *out = Offsets{};
+  out->marked = (h[0] & kOffsetsMarked) != 0;
+  if (h[0] & kOffsetsIrregular) return CGHIP_OK;
+  out->count = 0;
+  for (int k = 1; k <= kDiaMax; k++)
+    if (h[k] != INT32_MIN) out->off[out->count++] = h[k];
+  std::sort(out->off, out->off + out->count);
+  return CGHIP_OK;
+}
+
+// The symmetric diagonals of an uploaded matrix, if it has them: every
+// off-diagonal offset mirrored, at most kSym64Pairs pairs, every entry equal
+// to its transpose.  Not built (no error) otherwise, or where the device has
+// no memory left for them.
+template <typename M>
+int build_sym(cghip_ctx *c, const M &A, const Offsets &o, Sym64 *out) {
+  const int m = o.count;
+  if (m <= 0 || m % 2 != 0 || m > 2 * kSym64Pairs || o.marked || !sym64_fits(A.n)) return CGHIP_OK;
+  for (int k = 0; k < m; k++)
+    if (o.off[k] != -o.off[m - 1 - k]) return CGHIP_OK;
+  Sym64 S{};
+  S.n = A.n;
+  S.pairs = m / 2;
+  for (int k = 0; k < S.pairs; k++) S.off[k] = o.off[S.pairs + k];
+  int *found = reinterpret_cast<int *>(c->partial);
+  double *diag = nullptr, *up = nullptr;
+  const size_t streams = (size_t)S.pairs * ((size_t)A.n + kSym64Pad);
+  if (hipMalloc((void **)&diag, sizeof(double) * (size_t)A.n) != hipSuccess ||
+      hipMalloc((void **)&up, sizeof(double) * streams) != hipSuccess) {
+    (void)hipGetLastError();
+    if (diag) (void)hipFree(diag);
+    return CGHIP_OK;
+  }
+  S.diag = diag;
+  S.up = up;
+  int bad = 1;
+  hipError_t e = hipMemsetAsync(found, 0, sizeof(int), c->stream);
+  if (e == hipSuccess) e = sym64_build(A, S, diag, up, found, c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(&bad, found, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess || bad) free_sym(S);
+  HIPCHK(c, e);
+  *out = S;
   return CGHIP_OK;
 }
 
@@ -422,28 +507,6 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
   for (int e = 0; e < nnz; e++)
     if (index[e] < 0 || index[e] >= n)
       return fail(c, CGHIP_ERR_ARG, "CRS column index %d out of range at entry %d", index[e], e);
-  // distinct off-diagonal offsets j - i (ascending), for the DIA layout
-  int ndiag = 0;
-  int off[kDiaMax + 1];
-  for (int i = 0; i < n && ndiag >= 0; i++)
-    for (int e = ptr[i]; e < ptr[i + 1]; e++) {
-      if (e > ptr[i] && index[e] <= index[e - 1]) {
-        ndiag = -1;  // columns not ascending: the DIA order would differ
-        break;
-      }
-      const int o = index[e] - i;
-      if (o == 0) continue;
-      int d = 0;
-      while (d < ndiag && off[d] < o) d++;
-      if (d < ndiag && off[d] == o) continue;
-      if (ndiag == kDiaMax) {
-        ndiag = -1;
-        break;
-      }
-      for (int k = ndiag; k > d; k--) off[k] = off[k - 1];
-      off[d] = o;
-      ndiag++;
-    }
   if (c->n != n)
     if (int rc = cghip_set_size(c, n)) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
@@ -473,8 +536,17 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
   c->crs_nnz = nnz;
   c->crs_nrb = nrb;
   c->crs_short = crs_short_rows(n, ptr, nrb);
-  c->dia_ndiag = ndiag;
-  for (int d = 0; d < kDiaMax; d++) c->dia_off[d] = d < ndiag ? off[d] : 0;
+  Offsets o;
+  rc = find_offsets(c, crs_of(c), &o);
+  // rows of up to kShortRow entries: row blocks are 256-row chunks, so the
+  // partials of <p, q> are the same
+  if (!rc && c->crs_short) rc = build_sym(c, crs_of(c), o, &c->crs_sym);
+  if (rc) {
+    free_crs(c);
+    return rc;
+  }
+  c->dia_ndiag = o.count;
+  std::copy(o.off, o.off + kDiaMax, c->dia_off);
   c->has_crs = true;
   if (!c->format) c->format = CGHIP_FORMAT_CRS;
   return CGHIP_OK;
@@ -517,6 +589,13 @@ int cghip_upload_ell(cghip_ctx *c, int n, int width, const int32_t *length, cons
     return e;
   }
   c->ell_width = width;
+  Offsets o;
+  rc = find_offsets(c, ell_of(c), &o);
+  if (!rc) rc = build_sym(c, ell_of(c), o, &c->ell_sym);
+  if (rc) {
+    free_ell(c);
+    return rc;
+  }
   c->has_ell = true;
   if (!c->format) c->format = CGHIP_FORMAT_ELL;
   return CGHIP_OK;
@@ -653,17 +732,20 @@ int enqueue_iteration(cghip_ctx *c, const double *C, History h, hipEvent_t *ev) 
   const int G = spmv_blocks(c);
   // G <= 256: the update folds the SpMV's partials itself (no group fold)
   const bool direct = G <= kBlock;
+  const bool nt = loop_streams(c->n, matrix_row_bytes(c));
   const Partials pq1{c->pq1, nullptr}, pq2{c->pq1 + G, nullptr};
   double *grp = direct ? nullptr : pq2.a;
-  if (c->format == CGHIP_FORMAT_CRS)
+  if (sym_of(c).pairs)
+    HIPCHK(c, pcg_matvec_dot_sym64(sym_of(c), p, q, pq1, grp, c->d_state, c->stream));
+  else if (c->format == CGHIP_FORMAT_CRS)
     HIPCHK(c, pcg_matvec_dot_crs(crs_of(c), p, q, pq1, grp, c->d_state, c->stream));
   else
     HIPCHK(c, pcg_matvec_dot_ell(ell_of(c), p, q, pq1, grp, c->d_state, c->stream));
   if (ev) HIPCHK(c, hipEventRecord(ev[1], c->stream));
   HIPCHK(c, pcg_update(c->n, direct ? -G : fold_groups(G), r, q, C, direct ? pq1 : pq2, pr_of(c),
-                       c->d_state, h, c->stream));
+                       c->d_state, h, nt, c->stream));
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
-  HIPCHK(c, pcg_xpay(c->n, x, p, r, C, pr_of(c), c->d_state, h, c->stream));
+  HIPCHK(c, pcg_xpay(c->n, x, p, r, C, pr_of(c), c->d_state, h, nt, c->stream));
   if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));
   return CGHIP_OK;
 }
@@ -1112,7 +1194,7 @@ int cghip_solve_mixed(cghip_ctx *c, const cghip_mixed_opts *o, cghip_mixed_info 
   auto refresh = [&](bool first) -> int {
     if (ev) HIPCHK(c, hipEventRecord(ev[0], c->stream));
     if (!first) HIPCHK(c, mp_accumulate(n, x64, y32, scale, c->stream));
-    HIPCHK(c, matvec_crs(crs_of(c), x64, q64, c->stream));
+    HIPCHK(c, launch_matvec(c, x64, q64));
     HIPCHK(c, mp_residual(n, k64, q64, r64, pt, c->stream));
     if (poly) {
       HIPCHK(c, mp_restart(n, r64, scale, r32, y32, p32, false, prr, c->stream));

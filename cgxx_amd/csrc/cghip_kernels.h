@@ -122,6 +122,37 @@ struct Ell {
   int unit;  // 1: implicit unit diagonal, y_i = x_i + (sum of the stored products)
 };
 
+// FP64 matrix whose off-diagonal entries lie on 1 to kSym64Pairs mirrored
+// pairs of diagonals (2D and 3D stencils) and equal their transposes bit for
+// bit: the diagonal and the upper diagonals only, beside the uploaded arrays.
+// Stream k of up (up + k (n + kSym64Pad)) holds entry (i, i + off[k]) at i, and row i
+// reads its lower entry (i, i - off[k]) at i - off[k]; an absent entry holds
+// kF64Absent and is skipped.  8 (1 + pairs) bytes per row instead of 12 per
+// entry; the products and their order are those of the uploaded rows.
+constexpr int kSym64Pairs = 3;
+// FP64 bits of a signalling NaN: a matrix that holds them keeps its arrays.
+constexpr uint64_t kF64Absent = 0x7FF0000000000001ull;
+struct Sym64 {
+  const double *diag, *up;
+  int n, pairs;  // pairs = 0: not built
+  int off[kSym64Pairs];
+};
+// An upper stream starts n + kSym64Pad elements after the one before: see
+// kSymPad.
+constexpr int kSym64Pad = 1088;
+// Whether the vector kernels of an FP64 loop load what they only read (q, C,
+// r) and x past the caches: only where the loop's arrays, the matrix with
+// matrix_bytes a row and five vectors, outgrow the 256 MB last-level cache.
+// Iteration on the symmetric diagonals of 128^3 (151 MB) 57 cached against
+// 66 us, 145 x 150 x 155 (243 MB) 82 against 95, 160^3 (295 MB) 116 against
+// 112, 256^3 481 against 429.
+inline bool loop_streams(int64_t n, int64_t matrix_bytes) {
+  return (matrix_bytes + 40) * n > (int64_t(1) << 28);
+}
+// 32-bit byte offsets address a stream.
+inline bool sym64_fits(int64_t n) { return 8 * n <= (1ll << 32); }
+
+
 // Row blocks of the CRS kernels: greedy, at most kRowsMax rows and at most
 // kNnzCap nonzeros, except that a block always takes its first row (a row
 // longer than kNnzCap is then streamed through LDS in chunks).
@@ -163,15 +194,33 @@ hipError_t pcg_matvec_dot_crs(const Crs<double> &A, const double *p, double *q, 
                               double *pq2, SolveState *st, hipStream_t s);
 hipError_t pcg_matvec_dot_ell(const Ell<double> &A, const double *p, double *q, Partials pq,
                               double *pq2, SolveState *st, hipStream_t s);
+// The same on the symmetric diagonals: same rows, same partials.
+hipError_t matvec_sym64(const Sym64 &A, const double *x, double *y, hipStream_t s);
+hipError_t pcg_matvec_dot_sym64(const Sym64 &A, const double *p, double *q, Partials pq,
+                                double *pq2, SolveState *st, hipStream_t s);
+// Diagonals of an uploaded matrix.  matrix_offsets: found[1 .. kDiaMax] the
+// distinct off-diagonal offsets in no order (INT32_MIN: none), found[0] the
+// flags kOffsetsIrregular (a row's columns do not ascend, or more than
+// kDiaMax offsets) and kOffsetsMarked (an entry is kF64Absent).  sym64_build
+// writes diag and up whole and sets found[0] = 1 (0 beforehand) if an entry
+// differs from its transpose or has none.
+constexpr int kOffsetsIrregular = 1, kOffsetsMarked = 2;
+hipError_t matrix_offsets(const Crs<double> &A, int *found, hipStream_t s);
+hipError_t matrix_offsets(const Ell<double> &A, int *found, hipStream_t s);
+hipError_t sym64_build(const Crs<double> &A, const Sym64 &S, double *diag, double *up, int *found,
+                       hipStream_t s);
+hipError_t sym64_build(const Ell<double> &A, const Sym64 &S, double *diag, double *up, int *found,
+                       hipStream_t s);
 // alpha = rho / <p,q>; r -= alpha q; partials of <r,r> and <r,Cr>.  <p,q>
 // from gpq > 0 group sums in pq.a, or (gpq = -G, G <= 256) from the G
 // block partials themselves, folded to the same bits as their one group.
 hipError_t pcg_update(int n, int gpq, double *r, const double *q, const double *C, Partials pq,
-                      Partials pr, SolveState *st, History h, hipStream_t s);
+                      Partials pr, SolveState *st, History h, bool nt, hipStream_t s);
 // x += alpha p (the old p: each p element is read once outside the SpMV);
 // stop test; p = C r + beta p unless converged
 hipError_t pcg_xpay(int n, double *x, double *p, const double *r, const double *C, Partials pr,
-                    SolveState *st, History h, hipStream_t s);
+                    SolveState *st, History h, bool nt,
+                    hipStream_t s);
 
 // ---- mixed precision: FP32 inner PCG with FP64 reliable updates ----------
 //

@@ -27,6 +27,8 @@
 
 #include "device_common.h"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace cghip {
@@ -91,6 +93,94 @@ __global__ __launch_bounds__(kBlock) void k_pcg_matvec_dot_ell(Ell<double> A, co
   const double t = ell_rowblock<double, double, true, O32>(A, p, q, blockIdx.x);
   const double bp = block_fold(t, lds);
   if (threadIdx.x == 0) pq.a[blockIdx.x] = bp;
+}
+
+// Chunk of kBlock rows that block b of the symmetric kernels takes, or -1.
+// Blocks are dispatched to the 8 XCDs round robin; each XCD gets a contiguous
+// eighth of the chunks, so that a row's neighbours along the nearer diagonals
+// are still in that XCD's L2 (chunks in dispatch order: 256^3 ELL iteration
+// 430 against 418 us; in strips of the planes on top: no difference).
+__device__ inline int sym64_chunk(int n, int b) {
+  const int nrb = ell_chunks(n), x = b & 7, per = (nrb + 7) >> 3;
+  const int q = x * per + (b >> 3);
+  return q < min(nrb, (x + 1) * per) ? q : -1;
+}
+
+// Row r of the symmetric diagonals: lower entries from the farthest, the
+// diagonal, the upper entries, added left to right from 0 -- the order of a
+// row with ascending columns.  Every load is issued before any is used: the
+// addresses are clamped into the streams, and an entry that is absent or
+// would lie outside the matrix is dropped by a select.  NT: the diagonal,
+// the only stream read once, is loaded non-temporally (sym64_launch).  Bound
+// by memory: 48 bytes a row with three pairs against 100 from the uploaded
+// arrays; 256^3 product in the loop 303 -> 186 us (5.1 TB/s of the 950 MB
+// that the counters show, 1.2 times the bytes it needs), 128^3 40 -> 17 us.
+template <int P, bool NT>
+__device__ inline double sym64_row(const Sym64 &A, const double *__restrict__ x, int r, double &xr) {
+  const char *xb = reinterpret_cast<const char *>(x);
+  auto at = [](const char *base, int i) {
+    return *reinterpret_cast<const double *>(base + (uint32_t)i * 8u);
+  };
+  double lo[P], hi[P], xl[P], xh[P];
+  const double d = NT ? __builtin_nontemporal_load(A.diag + r) : A.diag[r];
+  xr = at(xb, r);
+#pragma unroll
+  for (int k = 0; k < P; k++) {
+    const char *u = reinterpret_cast<const char *>(A.up + k * ((int64_t)A.n + kSym64Pad));
+    const int below = max(r - A.off[k], 0);
+    hi[k] = at(u, r);
+    lo[k] = at(u, below);
+    xl[k] = at(xb, below);
+    xh[k] = at(xb, min(r + A.off[k], A.n - 1));
+  }
+  auto live = [](double v) { return __builtin_bit_cast(uint64_t, v) != kF64Absent; };
+  double s = 0.0;
+#pragma unroll
+  for (int k = P - 1; k >= 0; k--) {
+    const double t = s + lo[k] * xl[k];
+    s = live(lo[k]) && r >= A.off[k] ? t : s;
+  }
+  {
+    const double t = s + d * xr;
+    s = live(d) ? t : s;
+  }
+#pragma unroll
+  for (int k = 0; k < P; k++) {
+    const double t = s + hi[k] * xh[k];
+    s = live(hi[k]) ? t : s;
+  }
+  return s;
+}
+
+template <int P, bool NT>
+__global__ __launch_bounds__(kBlock) void k_matvec_sym64(Sym64 A, const double *__restrict__ x,
+                                                         double *__restrict__ y) {
+  const int c = sym64_chunk(A.n, blockIdx.x);
+  const int r = c * kBlock + (int)threadIdx.x;
+  if (c < 0 || r >= A.n) return;
+  double xr;
+  y[r] = sym64_row<P, NT>(A, x, r, xr);
+}
+
+// One partial of <p,q> per chunk, as from k_pcg_matvec_dot_crs and _ell.
+template <int P, bool NT>
+__global__ __launch_bounds__(kBlock) void k_pcg_matvec_dot_sym64(Sym64 A, const double *__restrict__ p,
+                                                                 double *__restrict__ q, Partials pq,
+                                                                 SolveState *st) {
+  __shared__ double lds[4];
+  if (!begin_iteration(st)) return;
+  const int c = sym64_chunk(A.n, blockIdx.x);
+  if (c < 0) return;
+  const int r = c * kBlock + (int)threadIdx.x;
+  double t = 0.0;
+  if (r < A.n) {
+    double pr;
+    const double s = sym64_row<P, NT>(A, p, r, pr);
+    q[r] = s;
+    t = pr * s;
+  }
+  const double bp = block_fold(t, lds);
+  if (threadIdx.x == 0) pq.a[c] = bp;
 }
 
 // Group fold: block g folds partials g*256 .. g*256+255 (zero past G) into
@@ -326,7 +416,7 @@ __device__ inline void update_elem(double &rv, double qv, double cv, double na, 
 // and 0.0 + that sum is what folding the single group sum gives (a sum
 // with only zeros added, except that -0.0 becomes +0.0), so the bits are
 // those of the two-level fold.
-template <bool JAC>
+template <bool JAC, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_pcg_update(
     int n, int gpq, double *__restrict__ r, const double *__restrict__ q,
     const double *__restrict__ C, Partials ppq, Partials prr, SolveState *st, History h) {
@@ -351,8 +441,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     for (int u = 0; u < kUnroll; u++) {
       const int64_t j = P.q + u * P.T;
       rv[u] = v2(r)[j];
-      qv[u] = v2_stream(q, j);
-      if (JAC) cv[u] = v2_stream(C, j);
+      qv[u] = NT ? v2_stream(q, j) : v2(q)[j];
+      if (JAC) cv[u] = NT ? v2_stream(C, j) : v2(C)[j];
     }
 #pragma unroll
     for (int u = 0; u < kUnroll; u++) {
@@ -380,7 +470,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 // the stop test (CG.cpp:344-355); if not converged rho = <r,z>,
 // b = rho / rho_old (CG.cpp:357-370) and p = z + b p with z = C o r
 // recomputed (CG.cpp:375-381).  Writes `next`.
-template <bool JAC>
+template <bool JAC, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_pcg_xpay(
     int n, double *__restrict__ x, double *__restrict__ p, const double *__restrict__ r,
     const double *__restrict__ C, Partials prr, SolveState *st, History h) {
@@ -430,10 +520,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
 #pragma unroll
     for (int u = 0; u < U; u++) {
       const int64_t j = P.q + u * P.T;
-      xv[u] = v2_stream(x, j);
+      xv[u] = NT ? v2_stream(x, j) : v2(x)[j];
       pv[u] = v2(p)[j];
-      rv[u] = v2_stream(r, j);
-      if (JAC) cv[u] = v2_stream(C, j);
+      rv[u] = NT ? v2_stream(r, j) : v2(r)[j];
+      if (JAC) cv[u] = NT ? v2_stream(C, j) : v2(C)[j];
     }
 #pragma unroll
     for (int u = 0; u < U; u++) {
@@ -444,7 +534,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
       const double zy = JAC ? cv[u].y * rv[u].y : rv[u].y;
       pv[u].x = zx + b * pv[u].x;
       pv[u].y = zy + b * pv[u].y;
-      v2_store_stream(x, j, xv[u]);
+      if (NT)
+        v2_store_stream(x, j, xv[u]);
+      else
+        v2(x)[j] = xv[u];
       v2(p)[j] = pv[u];
     }
   }
@@ -586,23 +679,66 @@ hipError_t pcg_matvec_dot_ell(const Ell<double> &A, const double *p, double *q, 
   return hipGetLastError();
 }
 
+// f(grid, pairs, non-temporal diagonal) of the symmetric kernels.  The
+// diagonal is streamed past the caches once a product's own bytes, 8 (3 +
+// pairs) a row, outgrow the 256 MB last-level cache: FP64 iteration at 160^3
+// 102.7 cached against 111.2 us, at 180^3 159 against 152, at 256^3 438
+// against 418.
+template <typename F>
+static hipError_t sym64_launch(const Sym64 &A, F f) {
+  if (A.pairs < 1 || A.pairs > kSym64Pairs) return hipErrorInvalidValue;
+  const dim3 grid(8 * ((ell_chunks(A.n) + 7) / 8));
+  const bool nt = 8 * (3 + (int64_t)A.pairs) * A.n > (int64_t(1) << 28);
+  auto pick = [&](auto pairs) {
+    nt ? f(grid, pairs, std::true_type()) : f(grid, pairs, std::false_type());
+  };
+  switch (A.pairs) {
+    case 1: pick(std::integral_constant<int, 1>()); break;
+    case 2: pick(std::integral_constant<int, 2>()); break;
+    default: pick(std::integral_constant<int, 3>()); break;
+  }
+  return hipGetLastError();
+}
+
+hipError_t matvec_sym64(const Sym64 &A, const double *x, double *y, hipStream_t s) {
+  return sym64_launch(A, [&](dim3 grid, auto p, auto nt) {
+    hipLaunchKernelGGL((k_matvec_sym64<p(), nt()>), grid, dim3(kBlock), 0, s, A, x, y);
+  });
+}
+
+hipError_t pcg_matvec_dot_sym64(const Sym64 &A, const double *p, double *q, Partials pq,
+                                double *pq2, SolveState *st, hipStream_t s) {
+  const hipError_t e = sym64_launch(A, [&](dim3 grid, auto pairs, auto nt) {
+    hipLaunchKernelGGL((k_pcg_matvec_dot_sym64<pairs(), nt()>), grid, dim3(kBlock), 0, s, A, p, q,
+                       pq, st);
+  });
+  const int G = ell_chunks(A.n);
+  if (e == hipSuccess && pq2)
+    hipLaunchKernelGGL(k_fold_groups, dim3(fold_groups(G)), dim3(kBlock), 0, s, pq.a, G, pq2);
+  return e == hipSuccess ? hipGetLastError() : e;
+}
+
 hipError_t pcg_update(int n, int gpq, double *r, const double *q, const double *C, Partials pq,
-                      Partials pr, SolveState *st, History h, hipStream_t s) {
+                      Partials pr, SolveState *st, History h, bool nt, hipStream_t s) {
+  auto launch = [&](auto k) {
+    hipLaunchKernelGGL(k, vgrid(n), dim3(kBlock), 0, s, n, gpq, r, q, C, pq, pr, st, h);
+  };
   if (C)
-    hipLaunchKernelGGL(k_pcg_update<true>, vgrid(n), dim3(kBlock), 0, s, n, gpq, r, q, C, pq, pr,
-                       st, h);
+    nt ? launch(k_pcg_update<true, true>) : launch(k_pcg_update<true, false>);
   else
-    hipLaunchKernelGGL(k_pcg_update<false>, vgrid(n), dim3(kBlock), 0, s, n, gpq, r, q, C, pq, pr,
-                       st, h);
+    nt ? launch(k_pcg_update<false, true>) : launch(k_pcg_update<false, false>);
   return hipGetLastError();
 }
 
 hipError_t pcg_xpay(int n, double *x, double *p, const double *r, const double *C, Partials pr,
-                    SolveState *st, History h, hipStream_t s) {
+                    SolveState *st, History h, bool nt, hipStream_t s) {
+  auto launch = [&](auto k) {
+    hipLaunchKernelGGL(k, vgrid(n), dim3(kBlock), 0, s, n, x, p, r, C, pr, st, h);
+  };
   if (C)
-    hipLaunchKernelGGL(k_pcg_xpay<true>, vgrid(n), dim3(kBlock), 0, s, n, x, p, r, C, pr, st, h);
+    nt ? launch(k_pcg_xpay<true, true>) : launch(k_pcg_xpay<true, false>);
   else
-    hipLaunchKernelGGL(k_pcg_xpay<false>, vgrid(n), dim3(kBlock), 0, s, n, x, p, r, C, pr, st, h);
+    nt ? launch(k_pcg_xpay<false, true>) : launch(k_pcg_xpay<false, false>);
   return hipGetLastError();
 }
 
