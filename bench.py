@@ -95,7 +95,10 @@ def algorithmic_bytes(short: str, meta: dict):
     table = [("k_pcg_matvec_dot_crs", crs_bytes(n, nnz, 8, 8)), ("k_matvec_crs<double", crs_bytes(n, nnz, 8, 8)),
              ("k_pcg_matvec_dot_ell", ell_bytes(n, nnz, 8, 8)), ("k_matvec_ell<double", ell_bytes(n, nnz, 8, 8)),
              ("k_pcg_update<true>", 32 * n), ("k_pcg_update<false>", 24 * n), ("k_pcg_xpay<true>", 48 * n),
-             ("k_pcg_xpay<false>", 40 * n), ("k_mp_matvec_dot<2>", 4 * D * n + 8 * n),
+             ("k_pcg_xpay<false>", 40 * n), ("k_mp_matvec_dot<2, true", 2 * D * n + 8 * n),
+             ("k_mp_matvec_dot_quad", 2 * D * n + 8 * n), ("k_mp_matvec_dot<2", 4 * D * n + 8 * n),
+             ("k_poly_quad<1,", D * n + 8 * n), ("k_poly_quad<2,", D * n + 12 * n),
+             ("k_poly_quad<0,", D * n + 16 * n), ("k_poly_quad_dot<0,", D * n + 16 * n),
              ("k_mp_update", 12 * n), ("k_mp_xpay_poly", 20 * n), ("k_mp_xpay", 20 * n),
              ("k_poly_step<false, 2, 1,", rec + 8 * n),
              ("k_poly_step<false, 2, 2,", rec + 12 * n),

@@ -100,7 +100,9 @@ struct cghip_ctx {
   bool dia_nd = false;
   float *dia_val = nullptr;
   uint16_t *dia_val16 = nullptr;  // FP16 copy for the polynomial's Clenshaw steps
+  bool dia_sym32 = false;         // Dia::sym32
   uint16_t *dia_up16 = nullptr;   // its upper diagonals when symmetric (Dia::up16), or null
+  int pad32 = 0;  // Dia::pad of v32, w32 and dia_up16
   float *v32[4] = {};
   MixedState *d_mstate = nullptr;
   MixedState *h_mstate = nullptr;  // pinned
@@ -159,6 +161,20 @@ int dalloc(cghip_ctx *c, T **p, size_t count) {
   return CGHIP_OK;
 }
 
+// The same with `pad` elements before and after (Dia::pad); freed by pfree.
+template <typename T>
+int palloc(cghip_ctx *c, T **p, size_t count, int pad) {
+  if (int rc = dalloc(c, p, count + 2 * (size_t)pad)) return rc;
+  *p += pad;
+  return CGHIP_OK;
+}
+
+template <typename T>
+void pfree(T *&p, int pad) {
+  if (p) (void)hipFree((void *)(p - pad));
+  p = nullptr;
+}
+
 template <typename T>
 void dfree(T *&p) {
   if (p) (void)hipFree((void *)p);
@@ -188,12 +204,14 @@ void free_fp32(cghip_ctx *c) {
   dfree(c->ell_slot_nd);
   dfree(c->dia_val);
   dfree(c->dia_val16);
-  dfree(c->dia_up16);
+  pfree(c->dia_up16, c->pad32);
   c->dia_nd = false;
+  c->dia_sym32 = false;
   c->ell_nd = false;
   c->ell_w_nd = 0;
-  for (auto &v : c->v32) dfree(v);
-  for (auto &v : c->w32) dfree(v);
+  for (auto &v : c->v32) pfree(v, c->pad32);
+  for (auto &v : c->w32) pfree(v, c->pad32);
+  c->pad32 = 0;
   c->has_scaled = false;
   c->nnz_nd = c->nrb_nd = c->short_nd = 0;
   c->has_fp32 = false;
@@ -264,7 +282,7 @@ Ell<double> ell_of(cghip_ctx *c) {
 
 Dia dia_of(cghip_ctx *c) {
   Dia d{c->dia_val, c->dia_val16, c->n, c->dia_ndiag > 0 ? c->dia_ndiag : 0, {}, 1, 0, 0,
-        c->dia_up16};
+        c->dia_up16, c->dia_sym32, c->pad32};
   for (int k = 0; k < kDiaMax; k++) d.off[k] = c->dia_off[k];
   dia_strips(d);
   return d;
@@ -925,9 +943,10 @@ int cghip_prepare_fp32(cghip_ctx *c) {
   drop_graph(c);
   free_fp32(c);
   const int n = c->n;
+  c->pad32 = quad_pad(dia_of(c));
   int rc = dalloc(c, &c->value32, (size_t)c->crs_nnz);
   for (auto &v : c->v32)
-    if (!rc) rc = dalloc(c, &v, (size_t)n);
+    if (!rc) rc = palloc(c, &v, (size_t)n, c->pad32);
   if (!rc) rc = dalloc(c, &c->scale64, (size_t)n);
   if (!rc && !c->d_mstate) rc = dalloc(c, &c->d_mstate, 1);
   if (!rc && !c->h_mstate) {
@@ -972,7 +991,8 @@ int cghip_prepare_fp32(cghip_ctx *c) {
     int w = 0;
     for (int i = 0; i < n; i++) w = std::max(w, ptr[i + 1] - ptr[i]);
     if (c->dia_ndiag > 0 && dia_pays(c->dia_ndiag, n, c->nnz_nd)) {
-      const size_t slots = (size_t)c->dia_ndiag * (size_t)n;
+      // a tile past the last stream: rows of a quad past the last row
+      const size_t slots = (size_t)c->dia_ndiag * (size_t)n + (c->pad32 ? kQuadTile : 0);
       rc = dalloc(c, &c->dia_val, slots);
       if (!rc) rc = dalloc(c, &c->dia_val16, 2 * (size_t)half_words(c->dia_ndiag) * (size_t)n);
       if (rc) {
@@ -992,22 +1012,24 @@ int cghip_prepare_fp32(cghip_ctx *c) {
         dfree(c->dia_val16);
         c->dia_nd = false;
       } else if (c->dia_ndiag == 2 * kSymPairs && dia_mirrored(dia_of(c))) {
-        // symmetric FP16 storage, kept only if every value equals its
-        // transpose's bit for bit
-        rc = dalloc(c, &c->dia_up16, (size_t)kSymPairs * ((size_t)n + kSymPad));
+        // symmetric storage, FP16 and FP32, used only if every value equals
+        // its transpose's bit for bit
+        rc = palloc(c, &c->dia_up16, (size_t)kSymPairs * ((size_t)n + kSymPad), c->pad32);
         if (rc) {
           free_fp32(c);
           return rc;
         }
         int *d_mis = reinterpret_cast<int *>(c->dot_out);
-        HIPCHK(c, hipMemsetAsync(d_mis, 0, sizeof(int), c->stream));
+        HIPCHK(c, hipMemsetAsync(d_mis, 0, 2 * sizeof(int), c->stream));
         Dia d = dia_of(c);
         d.up16 = nullptr;
         HIPCHK(c, dia_upper16(d, c->dia_up16, d_mis, c->stream));
-        int mis = 0;
-        HIPCHK(c, hipMemcpyAsync(&mis, d_mis, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, dia_symmetric32(d, d_mis + 1, c->stream));
+        int mis[2] = {1, 1};
+        HIPCHK(c, hipMemcpyAsync(mis, d_mis, sizeof(mis), hipMemcpyDeviceToHost, c->stream));
         if (int r = sync(c)) return r;
-        if (mis) dfree(c->dia_up16);
+        if (mis[0]) pfree(c->dia_up16, c->pad32);
+        c->dia_sym32 = !mis[1];
       }
     }
     if (!c->dia_nd && ell_pays(w, n, c->nnz_nd)) {
@@ -1101,7 +1123,7 @@ int cghip_set_poly(cghip_ctx *c, int degree, const double *coeffs, double b) {
   HIPCHK(c, hipStreamSynchronize(c->stream));
   for (auto &v : c->w32)
     if (!v)
-      if (int rc = dalloc(c, &v, (size_t)c->n)) return rc;
+      if (int rc = palloc(c, &v, (size_t)c->n, c->pad32)) return rc;
   HIPCHK(c, hipMemcpyAsync(c->d_poly, &pp, sizeof(PolyParams), hipMemcpyHostToDevice, c->stream));
   if (int r = sync(c)) return r;
   c->poly_degree = degree;
@@ -1421,7 +1443,8 @@ int cghip_mixed_iteration_bytes(const cghip_ctx *c, int precond, double *bytes) 
   // operator stream of one SpMV: FP32 values in the CG SpMV (DIA: one
   // stream per diagonal, no mask); the Clenshaw steps read DIA's FP16 row
   // records, or with symmetric storage its upper diagonals (2 bytes per
-  // stored pair; the lower values are those of earlier rows)
+  // stored pair; the lower values are those of earlier rows).  A product that
+  // reads the upper FP32 diagonals only (Dia::sym32) moves half of op32
   const double op32 = c->dia_nd ? 4.0 * d * n : c->ell_nd ? 8.0 * nnz + 4.0 * n
                                                           : 8.0 * nnz + 4.0 * (n + 1);
   const double op16 = !(c->dia_nd && c->poly_fp16) ? op32

@@ -332,6 +332,14 @@ struct Dia {
   // / 2 + k]), so the Clenshaw steps load 2 bytes per stored pair instead of
   // 4 and form the same products in the same order.
   const uint16_t *up16;
+  // 1: the same holds for the FP32 values of val (dia_symmetric32): the CG
+  // product reads its upper diagonals only, lower entries as those of rows
+  // i - o: 12 instead of 24 bytes a row.
+  int sym32;
+  // Elements that the FP32 vectors of the mixed loop and up16 have before
+  // row 0, and the vectors past row n - 1: the four-rows-per-thread kernels
+  // (quad_pad) then load every neighbour without a clamp.  0: a row per thread.
+  int pad;
 };
 // Diagonal pairs of the symmetric FP16 storage the Clenshaw steps read:
 // those of a 3D 7-point stencil.  A compile-time count keeps the row's
@@ -373,6 +381,20 @@ inline void dia_strips(Dia &d) {
   while (pc % w) w--;
   d.plane_chunks = pc;
   d.strip_chunks = w;
+}
+// Dia::pad of an operator: 0, or its farthest offset and one tile of 1,024 rows.
+// Four rows per thread need the mirrored pairs, and pay from where the dot
+// kernels' blocks walk more than one chunk: below, a quarter of the waves is
+// too few to cover the latency (64^3 step 3.4 us with a row per thread, 3.7
+// with four; CG product 8.1 against 9.7).  Offsets above n / 8 would pad the
+// vectors by more than a quarter.
+constexpr int kQuadTile = 1024;
+inline int quad_pad(const Dia &d) {
+  if (d.ndiag != 2 * kSymPairs || !dia_mirrored(d)) return 0;
+  const int64_t far = d.off[d.ndiag - 1];
+  if (((int64_t)d.n + kBlock - 1) / kBlock <= kDiaGMax || 8 * far > d.n) return 0;
+  const int64_t pad = (far + 63) / 64 * 64 + kQuadTile;
+  return 4 * ((int64_t)d.n + 2 * pad) <= (1ll << 32) ? (int)pad : 0;
 }
 inline bool dia_fits(int64_t ndiag, int64_t n) {
   return ndiag >= 1 && ndiag <= kDiaMax && ndiag * n * 4 <= (1ll << 32) && n * 4 <= (1ll << 32);
@@ -426,6 +448,9 @@ hipError_t scaled_dia(const Crs<double> &A, const double *s, const Dia &D, float
 // differs from its transpose's or a lower value lies outside the matrix:
 // up16 must then not be used.
 hipError_t dia_upper16(const Dia &D, uint16_t *up16, int *mismatch, hipStream_t st);
+// mismatch[0] = 1 (zeroed by the caller) if an FP32 value of a mirrored D
+// differs from its transpose's (Dia::sym32 must then stay 0).
+hipError_t dia_symmetric32(const Dia &D, int *mismatch, hipStream_t st);
 // x64 += scale o (double)y32 (scale nullable: plain add)
 hipError_t mp_accumulate(int n, double *x64, const float *y32, const double *scale, hipStream_t s);
 // r64 = k - q64; partials.a = ||r64||^2 (pairs order)

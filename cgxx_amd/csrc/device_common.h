@@ -5,6 +5,8 @@
 
 #include "cghip_kernels.h"
 
+#include <type_traits>
+
 #pragma clang fp contract(off)
 
 namespace cghip {
@@ -379,7 +381,7 @@ __device__ inline double ell_row_pre_epi(const EllPacked &A, const float *__rest
 // Clenshaw step 83.2 -> 75.9 us (the absent mark alone, per-diagonal
 // streams kept: 78.5 us; the record read as three 4-byte loads: 97.4 us).
 //
-// SYM (HALF only, Dia::up16 set, kSymPairs diagonal pairs): slot k holds
+// SYM (Dia::up16 set, or for FP32 values Dia::sym32; kSymPairs diagonal pairs): slot k holds
 // upper stream k at r and slot kSymPairs + k the same stream at r - o (row
 // r's value on the mirrored lower diagonal), each with x at its column; the
 // products are added in the stored order (lower diagonals from the
@@ -410,17 +412,20 @@ __device__ inline auto dia_row_load(const Dia &A, const float *__restrict__ x, i
     // then replaced by the absent mark); up16 is not streamed
     // non-temporally: rows r + o read it again
     constexpr int Q = kSymPairs;
-    const char *ub = reinterpret_cast<const char *>(A.up16);
-    const uint32_t nb = ((uint32_t)A.n + (uint32_t)kSymPad) * 2u;
+    typedef typename std::conditional<HALF, uint16_t, uint32_t>::type V;
+    constexpr uint32_t B = sizeof(V);
+    const char *ub = HALF ? reinterpret_cast<const char *>(A.up16)
+                          : reinterpret_cast<const char *>(A.val) + (int64_t)Q * A.n * 4;
+    const int64_t nb = HALF ? ((int64_t)A.n + kSymPad) * 2 : (int64_t)A.n * 4;
 #pragma unroll
     for (int k = 0; k < Q; k++) {
       const int o = A.off[Q + k];
       const int rl = max(r - o, 0);
-      const char *sk = ub + (uint32_t)k * nb;
-      const uint16_t up = *reinterpret_cast<const uint16_t *>(sk + (uint32_t)r * 2u);
-      const uint16_t lo = *reinterpret_cast<const uint16_t *>(sk + (uint32_t)rl * 2u);
+      const char *sk = ub + k * nb;
+      const V up = *reinterpret_cast<const V *>(sk + (uint32_t)r * B);
+      const V lo = *reinterpret_cast<const V *>(sk + (uint32_t)rl * B);
       l.v[k] = up;
-      l.v[Q + k] = r >= o ? lo : kHalfAbsent;
+      l.v[Q + k] = r >= o ? lo : HALF ? (V)kHalfAbsent : (V)kF32Absent;
       l.xv[k] = *reinterpret_cast<const float *>(xb + (uint32_t)min(r + o, last) * 4u);
       l.xv[Q + k] = *reinterpret_cast<const float *>(xb + (uint32_t)rl * 4u);
     }
@@ -467,14 +472,17 @@ __device__ inline double dia_row_finish(const Dia &A, int r, const L &l, Epi epi
   float s = 0.0f;
   if (SYM) {
     constexpr int Q = kSymPairs;
+    auto add = [&](int k) {
+      if (l.v[k] != (HALF ? kHalfAbsent : kF32Absent)) {
+        const float a = HALF ? (float)__builtin_bit_cast(_Float16, (uint16_t)l.v[k])
+                             : __uint_as_float(l.v[k]);
+        s += a * xf(l.xv[k]);
+      }
+    };
 #pragma unroll
-    for (int k = Q - 1; k >= 0; k--)
-      if (l.v[Q + k] != kHalfAbsent)
-        s += (float)__builtin_bit_cast(_Float16, (uint16_t)l.v[Q + k]) * xf(l.xv[Q + k]);
+    for (int k = Q - 1; k >= 0; k--) add(Q + k);
 #pragma unroll
-    for (int k = 0; k < Q; k++)
-      if (l.v[k] != kHalfAbsent)
-        s += (float)__builtin_bit_cast(_Float16, (uint16_t)l.v[k]) * xf(l.xv[k]);
+    for (int k = 0; k < Q; k++) add(k);
     return epi(r, s, l.pv);
   }
 #pragma unroll
@@ -492,6 +500,146 @@ __device__ inline double dia_row_pre_epi(const Dia &A, const float *__restrict__
                                          Epi epi, XF xf = XF()) {
   const auto l = dia_row_load<HALF, SYM>(A, x, r, pre);
   return dia_row_finish<HALF, SYM>(A, r, l, epi, xf);
+}
+
+// ---------------------------------------------------------------------------
+// Four consecutive rows per thread of a DIA operator whose kSymPairs mirrored
+// pairs of diagonals equal their transposes bit for bit: V = uint16_t reads
+// the streams Dia::up16, V = uint32_t the upper diagonals of Dia::val; row
+// i's lower entries are those of rows i - o.  G neighbouring lanes (64 or 16)
+// hold 4 G consecutive rows.  A row's products and their order are those of
+// dia_row_finish.
+
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef uint16_t h4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+// the same at an address aligned to its elements only
+typedef f4 f4_any __attribute__((aligned(4)));
+typedef h4 h4_any __attribute__((aligned(2)));
+typedef u4 u4_any __attribute__((aligned(4)));
+
+template <typename V>
+struct QuadOf;
+template <>
+struct QuadOf<uint16_t> {
+  typedef h4 vec;
+  typedef h4_any any;
+};
+template <>
+struct QuadOf<uint32_t> {
+  typedef u4 vec;
+  typedef u4_any any;
+};
+
+// The value of the lane before (after) of a group of G lanes, `edge` in its
+// first (last) lane.  Every lane of the group is active.
+template <int G>
+__device__ inline uint32_t lane_before(uint32_t v, uint32_t edge) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, G == 64 ? 0x138 : 0x111, 0xf, 0xf,
+                                               false);
+}
+template <int G>
+__device__ inline uint32_t lane_after(uint32_t v, uint32_t edge) {
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, G == 64 ? 0x130 : 0x101, 0xf, 0xf,
+                                               false);
+}
+
+template <typename V>
+struct DiaQuad {
+  typename QuadOf<V>::vec up[kSymPairs], lo[kSymPairs];
+  f4 own, xl[kSymPairs], xh[kSymPairs];
+};
+
+// All loads of rows r0 .. r0 + 3 of the lane, the g-th of its group.  Dia::pad
+// keeps them inside the allocations for every row of a tile, those before row
+// 0 and past the last one too; what lies there is dropped: an upper entry
+// past the matrix is absent, and a lower one before it is marked absent here.
+// UNIT (the nearest pair is +-1): x at r +- 1 and its lower value come from
+// the thread's own quad and its neighbour lanes', and one load for the two
+// ends of the group, instead of three more quads.
+template <typename V, bool UNIT, int G>
+__device__ inline void dia_quad_load(const Dia &A, const float *__restrict__ x, int r0, int g,
+                                     DiaQuad<V> &l) {
+  typedef typename QuadOf<V>::any Any;
+  constexpr uint32_t B = sizeof(V);
+  constexpr int Q = kSymPairs;
+  const char *xb = reinterpret_cast<const char *>(x);
+  const char *ub = B == 2 ? reinterpret_cast<const char *>(A.up16)
+                          : reinterpret_cast<const char *>(A.val) + (int64_t)Q * A.n * 4;
+  const int64_t sb = B == 2 ? ((int64_t)A.n + kSymPad) * 2 : (int64_t)A.n * 4;
+  // byte offsets from pad elements before row 0: never negative
+  const char *up = ub - (int64_t)A.pad * B, *xp = xb - (int64_t)A.pad * 4;
+  auto at = [&](int i, uint32_t bytes) { return (uint32_t)(i + A.pad) * bytes; };
+  auto values = [&](int k, int i) {
+    return *reinterpret_cast<const Any *>(up + k * sb + at(i, B));
+  };
+  auto xs = [&](int i) { return *reinterpret_cast<const f4_any *>(xp + at(i, 4u)); };
+  l.own = xs(r0);
+#pragma unroll
+  for (int k = 0; k < Q; k++) {
+    const int o = A.off[Q + k];
+    l.up[k] = values(k, r0);
+    if (UNIT && k == 0) continue;
+    l.lo[k] = values(k, r0 - o);
+    l.xl[k] = xs(r0 - o);
+    l.xh[k] = xs(r0 + o);
+  }
+  if (UNIT) {
+    const int before = r0 - 4 * g - 1;
+    const uint32_t xe = *reinterpret_cast<const uint32_t *>(xp + at(g == G - 1 ? r0 + 4 : before, 4u));
+    const uint32_t le = *reinterpret_cast<const V *>(up + at(before, B));
+    const uint32_t xa = lane_before<G>(__float_as_uint(l.own.w), xe);
+    const uint32_t xz = lane_after<G>(__float_as_uint(l.own.x), xe);
+    l.xl[0] = f4{__uint_as_float(xa), l.own.x, l.own.y, l.own.z};
+    l.xh[0] = f4{l.own.y, l.own.z, l.own.w, __uint_as_float(xz)};
+    l.lo[0].x = (V)lane_before<G>((uint32_t)l.up[0].w, le);
+    l.lo[0].y = l.up[0].x;
+    l.lo[0].z = l.up[0].y;
+    l.lo[0].w = l.up[0].z;
+  }
+  if (r0 < A.off[2 * Q - 1]) {
+#pragma unroll
+    for (int k = 0; k < Q; k++)
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        if (r0 + e < A.off[Q + k]) l.lo[k][e] = B == 2 ? (V)kHalfAbsent : (V)kF32Absent;
+  }
+}
+
+// Sum of the stored products of row e (0 .. 3) of the quad.
+template <typename V, typename XF = XIdent>
+__device__ inline float dia_quad_sum(const DiaQuad<V> &l, int e, XF xf = XF()) {
+  auto add = [&](float s, V v, float xv) {
+    const bool live = sizeof(V) == 2 ? v != (V)kHalfAbsent : v != (V)kF32Absent;
+    const float a = sizeof(V) == 2 ? (float)__builtin_bit_cast(_Float16, (uint16_t)v)
+                                   : __builtin_bit_cast(float, (uint32_t)v);
+    const float t = s + a * xf(xv);
+    return live ? t : s;
+  };
+  float s = 0.0f;
+#pragma unroll
+  for (int k = kSymPairs - 1; k >= 0; k--) s = add(s, l.lo[k][e], l.xl[k][e]);
+#pragma unroll
+  for (int k = 0; k < kSymPairs; k++) s = add(s, l.up[k][e], l.xh[k][e]);
+  return s;
+}
+
+// Tile of 4 chunks (1,024 rows) that block b of the quad kernels without a
+// dot takes, or -1: each XCD (blocks go to the 8 of them round robin) has a
+// contiguous eighth of the tiles, in the strip order of dia_strips where the
+// plane and its strips are whole tiles.
+__host__ __device__ inline int quad_tiles(int n) {
+  return (int)(((int64_t)n + kQuadTile - 1) / kQuadTile);
+}
+__device__ inline int quad_tile(const Dia &A, int b) {
+  const int nt = quad_tiles(A.n), x = b & 7, per = (nt + 7) >> 3;
+  const int q = x * per + (b >> 3);
+  if (q >= min(nt, (x + 1) * per)) return -1;
+  const int P = A.plane_chunks >> 2, W = A.strip_chunks >> 2;
+  if (W <= 0 || (A.plane_chunks & 3) || (A.strip_chunks & 3)) return q;
+  const int strip = (nt / P) * W;  // tiles of one strip over all planes
+  const int s = q / strip, rem = q - s * strip, z = rem / W;
+  return z * P + s * W + (rem - z * W);
 }
 
 // ELL rows rb*256 + t: y = A x; with WITH_DOT, returns the owner's
