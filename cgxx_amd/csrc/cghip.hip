@@ -62,6 +62,9 @@ struct cghip_ctx {
   double *pq1 = nullptr;
   size_t pq1_cap = 0;
   double *dot_out = nullptr;
+  // second buffer of P in the FP64 loop of two kernels; allocated by a solve
+  // that runs it
+  double *p_alt = nullptr;
 
   // solver
   SolveState *d_state = nullptr;
@@ -479,6 +482,7 @@ int cghip_destroy(cghip_ctx *c) {
   dfree(c->pq1);
   dfree(c->d_poly);
   dfree(c->dot_out);
+  dfree(c->p_alt);
   dfree(c->d_state);
   dfree(c->d_mstate);
   dfree(c->d_hist);
@@ -502,6 +506,7 @@ int cghip_set_size(cghip_ctx *c, int n) {
     free_fp32(c);
     free_ell(c);
     dfree(c->jac);
+    dfree(c->p_alt);
     c->has_jac = false;
     c->format = 0;
     c->n = 0;
@@ -748,8 +753,8 @@ int enqueue_iteration(cghip_ctx *c, const double *C, History h, hipEvent_t *ev) 
          *x = c->vec[CGHIP_VEC_X];
   if (ev) HIPCHK(c, hipEventRecord(ev[0], c->stream));
   const int G = spmv_blocks(c);
-  // G <= 256: the update folds the SpMV's partials itself (no group fold)
-  const bool direct = G <= kBlock;
+  // the update folds few SpMV partials itself (no group fold)
+  const bool direct = G <= kFoldDirect;
   const bool nt = loop_streams(c->n, matrix_row_bytes(c));
   const Partials pq1{c->pq1, nullptr}, pq2{c->pq1 + G, nullptr};
   double *grp = direct ? nullptr : pq2.a;
@@ -765,6 +770,30 @@ int enqueue_iteration(cghip_ctx *c, const double *C, History h, hipEvent_t *ev) 
   if (ev) HIPCHK(c, hipEventRecord(ev[2], c->stream));
   HIPCHK(c, pcg_xpay(c->n, x, p, r, C, pr_of(c), c->d_state, h, nt, c->stream));
   if (ev) HIPCHK(c, hipEventRecord(ev[3], c->stream));
+  return CGHIP_OK;
+}
+
+// Whether the loop runs two kernels an iteration (pcg_step_sym64).
+bool two_kernels(const cghip_ctx *c) {
+  return sym_of(c).pairs && ell_chunks(c->n) <= kSmallChunks;
+}
+
+// The first product of such a loop.
+int enqueue_first_product(cghip_ctx *c) {
+  HIPCHK(c, pcg_matvec_dot_sym64(sym_of(c), c->vec[CGHIP_VEC_P], c->vec[CGHIP_VEC_Q],
+                                 Partials{c->pq1, nullptr}, nullptr, c->d_state, c->stream));
+  return CGHIP_OK;
+}
+
+// One iteration of it: p in P before an even one, in p_alt before an odd one.
+int enqueue_two_kernels(cghip_ctx *c, const double *C, History h, bool odd) {
+  double *p = c->vec[CGHIP_VEC_P], *q = c->vec[CGHIP_VEC_Q], *r = c->vec[CGHIP_VEC_R],
+         *x = c->vec[CGHIP_VEC_X];
+  const Partials pq1{c->pq1, nullptr};
+  HIPCHK(c, pcg_update_small(c->n, ell_chunks(c->n), r, q, C, pq1, pr_of(c), c->d_state, h,
+                             c->stream));
+  HIPCHK(c, pcg_step_sym64(sym_of(c), x, odd ? c->p_alt : p, odd ? p : c->p_alt, q, r, C, pr_of(c),
+                           pq1, c->d_state, h, c->stream));
   return CGHIP_OK;
 }
 
@@ -842,6 +871,12 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
   int batch = o->batch > 0 ? o->batch : (c->n >= (1 << 20) ? 8 : 32);
   if (o->batch <= 0) batch = std::min(batch, o->max_iter);
   if (mode == CGHIP_PROFILE_KERNELS) batch = 1;
+  const bool two = mode == CGHIP_PROFILE_NONE && two_kernels(c);
+  if (two) {
+    batch += batch & 1;  // every batch starts with p in P
+    if (!c->p_alt)
+      if (int rc = dalloc(c, &c->p_alt, (size_t)c->n)) return rc;
+  }
   // events[0..1] bracket the set-up; events[2..5] the kernels of an iteration.
   if (mode != CGHIP_PROFILE_NONE && ensure_events(c, 6)) return CGHIP_ERR_HIP;
   hipEvent_t *ev = mode != CGHIP_PROFILE_NONE ? c->events.data() : nullptr;
@@ -873,6 +908,8 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
   HIPCHK(c, pcg_init(c->n, c->vec[CGHIP_VEC_K], c->vec[CGHIP_VEC_R], c->vec[CGHIP_VEC_P], C,
                      pr_of(c), c->d_state, h, c->stream));
   if (ev) HIPCHK(c, hipEventRecord(ev[1], c->stream));
+  if (two)
+    if (int rc = enqueue_first_product(c)) return rc;
   if (int rc = read_state()) return rc;
   if (ev) {
     info->ms_init = elapsed(ev[0], ev[1]);
@@ -894,7 +931,8 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
       hipGraph_t g = nullptr;
       HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
       int rc = CGHIP_OK;
-      for (int i = 0; i < batch && !rc; i++) rc = enqueue_iteration(c, C, h, nullptr);
+      for (int i = 0; i < batch && !rc; i++)
+        rc = two ? enqueue_two_kernels(c, C, h, i & 1) : enqueue_iteration(c, C, h, nullptr);
       hipError_t e = hipStreamEndCapture(c->stream, &g);
       if (rc) {
         if (g) (void)hipGraphDestroy(g);
@@ -920,7 +958,15 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
         return fail(c, CGHIP_ERR_STATE, "solver did not stop after %ld batches", nb);
       HIPCHK(c, hipGraphLaunch(c->graph, c->stream));
       if (int rc = read_state()) return rc;
-      if (c->h_state->cur.done || c->h_state->next.done) break;
+      const Scalars &nx = c->h_state->next;
+      if (c->h_state->cur.done || nx.done || (two && nx.iteration >= o->max_iter)) break;
+    }
+    // p changed its buffer in every iteration but a converging one
+    const Scalars &nx = c->h_state->next;
+    if (two && ((nx.iteration - (nx.residual <= o->tol ? 1 : 0)) & 1)) {
+      HIPCHK(c, hipMemcpyAsync(c->vec[CGHIP_VEC_P], c->p_alt, sizeof(double) * (size_t)c->n,
+                               hipMemcpyDeviceToDevice, c->stream));
+      if (int rc = sync(c)) return rc;
     }
   }
   const auto t1 = std::chrono::steady_clock::now();

@@ -52,6 +52,12 @@ inline int spmv_grid(int nrb) {
 // ELL kernels: 256-row chunks, one row per thread; the FP64 ones one block
 // per chunk, the FP32 ones at most 2048 blocks.
 __host__ __device__ inline int ell_chunks(int n) { return (int)(((int64_t)n + kBlock - 1) / kBlock); }
+// SpMV partials that the r update folds itself; more go through k_fold_groups
+// first, a launch of its own (594 partials: iteration 17.0 -> 15.7 us without).
+constexpr int kFoldDirect = 2048;
+// Systems of at most this many 256-row chunks run the loop of two kernels.
+constexpr int kSmallChunks = 1024;
+static_assert(kSmallChunks <= kFoldDirect, "the small update folds the partials itself");
 // Groups of 256 partials folded by k_fold_groups.
 inline int fold_groups(int G) { return (G + kBlock - 1) / kBlock; }
 inline int ell32_grid(int n) { return spmv_grid(ell_chunks(n)); }
@@ -188,7 +194,7 @@ hipError_t pcg_init(int n, const double *k, double *r, double *p, const double *
 // q = A p with one partial of <p,q> per row block (CRS) or 256-row chunk
 // (ELL) in pq.a, then (pq2 non-null) those partials folded in groups of
 // 256 into pq2[0 .. fold_groups(G)), G the number of row blocks / chunks.
-// With G <= 256 the loop passes pq2 = null and the update folds the G
+// With G <= kFoldDirect the loop passes pq2 = null and the update folds the G
 // partials itself (pcg_update with gpq = -G).
 hipError_t pcg_matvec_dot_crs(const Crs<double> &A, const double *p, double *q, Partials pq,
                               double *pq2, SolveState *st, hipStream_t s);
@@ -212,10 +218,19 @@ hipError_t sym64_build(const Crs<double> &A, const Sym64 &S, double *diag, doubl
 hipError_t sym64_build(const Ell<double> &A, const Sym64 &S, double *diag, double *up, int *found,
                        hipStream_t s);
 // alpha = rho / <p,q>; r -= alpha q; partials of <r,r> and <r,Cr>.  <p,q>
-// from gpq > 0 group sums in pq.a, or (gpq = -G, G <= 256) from the G
-// block partials themselves, folded to the same bits as their one group.
+// from gpq > 0 group sums in pq.a, or (gpq = -G, G <= kFoldDirect) from the G
+// block partials themselves, folded to the same bits.
 hipError_t pcg_update(int n, int gpq, double *r, const double *q, const double *C, Partials pq,
                       Partials pr, SolveState *st, History h, bool nt, hipStream_t s);
+// The loop of two kernels (n of at most kSmallChunks chunks): the update as
+// the iteration's first kernel, from the G SpMV partials; then pcg_xpay (the
+// new p into pnext) and the next pcg_matvec_dot_sym64 in one.  Values and
+// partials are those of the loop of three.
+hipError_t pcg_update_small(int n, int G, double *r, const double *q, const double *C, Partials pq,
+                            Partials pr, SolveState *st, History h, hipStream_t s);
+hipError_t pcg_step_sym64(const Sym64 &A, double *x, const double *p, double *pnext, double *q,
+                          const double *r, const double *C, Partials pr, Partials pq,
+                          SolveState *st, History h, hipStream_t s);
 // x += alpha p (the old p: each p element is read once outside the SpMV);
 // stop test; p = C r + beta p unless converged
 hipError_t pcg_xpay(int n, double *x, double *p, const double *r, const double *C, Partials pr,

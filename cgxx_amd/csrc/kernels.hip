@@ -106,6 +106,11 @@ __device__ inline int sym64_chunk(int n, int b) {
   return q < min(nrb, (x + 1) * per) ? q : -1;
 }
 
+// Element i of a vector of at most 2^32 bytes.
+__device__ inline double elem(const double *__restrict__ v, int i) {
+  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(v) + (uint32_t)i * 8u);
+}
+
 // Row r of the symmetric diagonals: lower entries from the farthest, the
 // diagonal, the upper entries, added left to right from 0 -- the order of a
 // row with ascending columns.  Every load is issued before any is used: the
@@ -115,41 +120,57 @@ __device__ inline int sym64_chunk(int n, int b) {
 // by memory: 48 bytes a row with three pairs against 100 from the uploaded
 // arrays; 256^3 product in the loop 303 -> 186 us (5.1 TB/s of the 950 MB
 // that the counters show, 1.2 times the bytes it needs), 128^3 40 -> 17 us.
-template <int P, bool NT>
-__device__ inline double sym64_row(const Sym64 &A, const double *__restrict__ x, int r, double &xr) {
-  const char *xb = reinterpret_cast<const char *>(x);
-  auto at = [](const char *base, int i) {
-    return *reinterpret_cast<const double *>(base + (uint32_t)i * 8u);
-  };
-  double lo[P], hi[P], xl[P], xh[P];
-  const double d = NT ? __builtin_nontemporal_load(A.diag + r) : A.diag[r];
-  xr = at(xb, r);
+template <int P>
+struct Sym64Loads {
+  double d, lo[P], hi[P];
+};
+
+template <int P, bool NT = false>
+__device__ inline void sym64_load(const Sym64 &A, int r, Sym64Loads<P> &l) {
+  l.d = NT ? __builtin_nontemporal_load(A.diag + r) : A.diag[r];
 #pragma unroll
   for (int k = 0; k < P; k++) {
-    const char *u = reinterpret_cast<const char *>(A.up + k * ((int64_t)A.n + kSym64Pad));
-    const int below = max(r - A.off[k], 0);
-    hi[k] = at(u, r);
-    lo[k] = at(u, below);
-    xl[k] = at(xb, below);
-    xh[k] = at(xb, min(r + A.off[k], A.n - 1));
+    const double *u = A.up + k * ((int64_t)A.n + kSym64Pad);
+    l.hi[k] = elem(u, r);
+    l.lo[k] = elem(u, max(r - A.off[k], 0));
   }
+}
+
+// xl, xh: x at r - off[k] and r + off[k].
+template <int P>
+__device__ inline double sym64_sum(const Sym64 &A, const Sym64Loads<P> &l, const double *xl,
+                                   const double *xh, double xr, int r) {
   auto live = [](double v) { return __builtin_bit_cast(uint64_t, v) != kF64Absent; };
   double s = 0.0;
 #pragma unroll
   for (int k = P - 1; k >= 0; k--) {
-    const double t = s + lo[k] * xl[k];
-    s = live(lo[k]) && r >= A.off[k] ? t : s;
+    const double t = s + l.lo[k] * xl[k];
+    s = live(l.lo[k]) && r >= A.off[k] ? t : s;
   }
   {
-    const double t = s + d * xr;
-    s = live(d) ? t : s;
+    const double t = s + l.d * xr;
+    s = live(l.d) ? t : s;
   }
 #pragma unroll
   for (int k = 0; k < P; k++) {
-    const double t = s + hi[k] * xh[k];
-    s = live(hi[k]) ? t : s;
+    const double t = s + l.hi[k] * xh[k];
+    s = live(l.hi[k]) ? t : s;
   }
   return s;
+}
+
+template <int P, bool NT>
+__device__ inline double sym64_row(const Sym64 &A, const double *__restrict__ x, int r, double &xr) {
+  Sym64Loads<P> l;
+  double xl[P], xh[P];
+  sym64_load<P, NT>(A, r, l);
+  xr = elem(x, r);
+#pragma unroll
+  for (int k = 0; k < P; k++) {
+    xl[k] = elem(x, max(r - A.off[k], 0));
+    xh[k] = elem(x, min(r + A.off[k], A.n - 1));
+  }
+  return sym64_sum<P>(A, l, xl, xh, xr, r);
 }
 
 template <int P, bool NT>
@@ -399,6 +420,31 @@ __global__ __launch_bounds__(kBlock) void k_pcg_init_finish(Partials pa, int G, 
   }
 }
 
+// Fold of G <= kFoldDirect partials as k_fold_groups and then fold_partials
+// over its group sums give it (adding 0.0 as they do), every load in flight
+// at once and one barrier.
+__device__ __forceinline__ double fold_two_levels(const double *__restrict__ partial, int G,
+                                         double (*lds)[4]) {
+  constexpr int M = kFoldDirect / kBlock;
+  const int t = threadIdx.x, lane = t & 63, groups = (G + kBlock - 1) / kBlock;
+  double v[M];
+#pragma unroll
+  for (int g = 0; g < M; g++) v[g] = partial[min(g * kBlock + t, G - 1)];
+#pragma unroll
+  for (int g = 0; g < M; g++) {
+    if (g < groups) {
+      const double w = wave_fold(g * kBlock + t < G ? v[g] : 0.0);
+      if (lane == 0) lds[g][t >> 6] = w;
+    }
+  }
+  __syncthreads();
+  const int g = min(lane, groups - 1);
+  const double sum = 0.0 + (((lds[g][0] + lds[g][1]) + lds[g][2]) + lds[g][3]);
+  const double w = wave_fold(lane < groups ? sum : 0.0);
+  __syncthreads();
+  return __shfl(w, 0, 64) + 0.0;
+}
+
 template <bool JAC>
 __device__ inline void update_elem(double &rv, double qv, double cv, double na, double &s_rr,
                                    double &s_rz) {
@@ -411,21 +457,18 @@ __device__ inline void update_elem(double &rv, double qv, double cv, double na, 
 // the x += a p of CG.cpp:340 is done by the last kernel, which reads p
 // anyway); partials of <r,r> and <r,z> with z = C o r (CG.cpp:344, 363-366).
 // gpq > 0: <p,q> folds the gpq group sums in ppq.a (k_fold_groups).
-// gpq = -G (G <= 256, small systems, one launch fewer per iteration): the
-// block folds the G SpMV partials as k_fold_groups folds its one group,
-// and 0.0 + that sum is what folding the single group sum gives (a sum
-// with only zeros added, except that -0.0 becomes +0.0), so the bits are
-// those of the two-level fold.
+// gpq = -G (G <= kFoldDirect, small systems, one launch fewer per iteration):
+// the block folds the G SpMV partials themselves, to the same bits.
 template <bool JAC, bool NT>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_pcg_update(
     int n, int gpq, double *__restrict__ r, const double *__restrict__ q,
     const double *__restrict__ C, Partials ppq, Partials prr, SolveState *st, History h) {
   __shared__ double lds[4];
+  __shared__ double lds2[kFoldDirect / kBlock][4];
   const Scalars c = st->cur;
   if (c.done) return;
   const double pq =
-      gpq > 0 ? fold_partials(ppq.a, gpq, lds)
-              : 0.0 + block_fold((int)threadIdx.x < -gpq ? ppq.a[threadIdx.x] : 0.0, lds);
+      gpq > 0 ? fold_partials(ppq.a, gpq, lds) : fold_two_levels(ppq.a, -gpq, lds2);
   const double a = c.rho / pq;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     st->alpha = a;
@@ -466,25 +509,12 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     prr.b[blockIdx.x] = b1;
   }
 }
-// Last kernel of an iteration: x += a p with the old p (CG.cpp:340); r2 and
-// the stop test (CG.cpp:344-355); if not converged rho = <r,z>,
-// b = rho / rho_old (CG.cpp:357-370) and p = z + b p with z = C o r
-// recomputed (CG.cpp:375-381).  Writes `next`.
-template <bool JAC, bool NT>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_pcg_xpay(
-    int n, double *__restrict__ x, double *__restrict__ p, const double *__restrict__ r,
-    const double *__restrict__ C, Partials prr, SolveState *st, History h) {
-  __shared__ double lds[4];
-  const Scalars c = st->cur;
-  if (c.done) return;
-  const int G = gridDim.x;  // the update kernel ran on the same grid
-  double r2, rz;
-  fold_partials2(prr.a, G, prr.b, G, lds, r2, rz);
+// End of iteration c: the stop test (CG.cpp:344-355), true if it converged;
+// block 0 writes `next` and the history.
+__device__ inline bool end_iteration(SolveState *st, const Scalars &c, double r2, double rho,
+                                     double b, const History &h) {
   const double res = sqrt(r2) / st->nrm2_0;
   const bool converged = res <= st->tol;
-  const double rho = JAC ? rz : r2;
-  const double b = rho / c.rho;
-  const double a = st->alpha;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     const int it = c.iteration;
     Scalars s = c;
@@ -505,6 +535,27 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     }
     st->next = s;
   }
+  return converged;
+}
+
+// Last kernel of an iteration: x += a p with the old p (CG.cpp:340); r2 and
+// the stop test (CG.cpp:344-355); if not converged rho = <r,z>,
+// b = rho / rho_old (CG.cpp:357-370) and p = z + b p with z = C o r
+// recomputed (CG.cpp:375-381).  Writes `next`.
+template <bool JAC, bool NT>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_pcg_xpay(
+    int n, double *__restrict__ x, double *__restrict__ p, const double *__restrict__ r,
+    const double *__restrict__ C, Partials prr, SolveState *st, History h) {
+  __shared__ double lds[4];
+  const Scalars c = st->cur;
+  if (c.done) return;
+  const int G = gridDim.x;  // the update kernel ran on the same grid
+  double r2, rz;
+  fold_partials2(prr.a, G, prr.b, G, lds, r2, rz);
+  const double rho = JAC ? rz : r2;
+  const double b = rho / c.rho;
+  const double a = st->alpha;
+  const bool converged = end_iteration(st, c, r2, rho, b, h);
   // x += a p always; p = z + b p unless the loop stops here.  Four streams
   // per element: unrolled twice to stay within 64 VGPRs.  x, r and C are
   // streamed non-temporally: only p stays cached for the next SpMV.
@@ -549,6 +600,145 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
       p[e] = ze + b * pe;
     }
   }
+}
+
+// ---------------------------------------------------------------------------
+// The loop of small systems on the symmetric diagonals: two kernels an
+// iteration instead of three.  Each kernel's time is its launch and one chain
+// of latencies (state and partials, fold, vectors, fold, store), so every load
+// is issued before the first fold, and a kernel of an iteration that is off
+// is told apart only where it would store.  Iteration with three kernels and
+// with two: 256 x 256 12.5 and 8.0 us (9.9 with the vectors loaded after the
+// fold), 61 x 47 x 53 15.6 and 11.8, 64^3 17.2 and 14.1; with more than a
+// chunk per block the neighbours' r, C and p cost more than the launch:
+// 80^3 26.5 and 27.5, 128^3 56 and 65.
+
+// Sums over the block of two values, as block_fold gives each; one barrier,
+// lds used once.
+__device__ inline void block_fold2(double &a, double &b, double (*lds)[4]) {
+  a = wave_fold(a);
+  b = wave_fold(b);
+  if ((threadIdx.x & 63) == 0) {
+    lds[0][threadIdx.x >> 6] = a;
+    lds[1][threadIdx.x >> 6] = b;
+  }
+  __syncthreads();
+  a = ((lds[0][0] + lds[0][1]) + lds[0][2]) + lds[0][3];
+  b = ((lds[1][0] + lds[1][1]) + lds[1][2]) + lds[1][3];
+}
+
+// k_pcg_update for at most one pair per thread, as the iteration's first
+// kernel: copies the loop scalars `next` -> `cur` and stops at CG_MAX_ITER
+// (CG.cpp:323).
+template <bool JAC>
+__global__ __launch_bounds__(kBlock) void k_pcg_update_small(int n, int G, double *__restrict__ r,
+                                                             const double *__restrict__ q,
+                                                             const double *__restrict__ C,
+                                                             const double *__restrict__ ppq,
+                                                             Partials prr, SolveState *st, History h) {
+  __shared__ double lds[2][4];
+  __shared__ double lds2[kFoldDirect / kBlock][4];
+  const int e = 2 * (blockIdx.x * kBlock + (int)threadIdx.x);
+  const int e0 = min(e, n - 1), e1 = min(e + 1, n - 1);
+  double r0 = r[e0], r1 = r[e1];
+  const double q0 = q[e0], q1 = q[e1];
+  const double c0 = JAC ? C[e0] : 0.0, c1 = JAC ? C[e1] : 0.0;
+  // field by field: as a struct it took stack, whose move to LDS reads the
+  // dispatch packet in host memory (12 us a kernel instead of 4)
+  const double rho = st->next.rho, r2 = st->next.r2, res = st->next.residual, beta = st->next.beta;
+  const int it = st->next.iteration;
+  const bool off = st->next.done || it >= st->max_iter;
+  const double pq = fold_two_levels(ppq, G, lds2);
+  const double a = rho / pq;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->cur.rho = rho;
+    st->cur.r2 = r2;
+    st->cur.residual = res;
+    st->cur.beta = beta;
+    st->cur.iteration = it;
+    st->cur.done = off;
+  }
+  if (off) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    st->alpha = a;
+    if (h.pq && it < h.cap) h.pq[it] = pq;
+    if (h.alpha && it < h.cap) h.alpha[it] = a;
+  }
+  double s_rr = 0.0, s_rz = 0.0;
+  if (e < n) {
+    update_elem<JAC>(r0, q0, c0, -a, s_rr, s_rz);
+    r[e] = r0;
+  }
+  if (e + 1 < n) {
+    update_elem<JAC>(r1, q1, c1, -a, s_rr, s_rz);
+    r[e + 1] = r1;
+  }
+  block_fold2(s_rr, s_rz, lds);
+  if (threadIdx.x == 0) {
+    prr.a[blockIdx.x] = s_rr;
+    prr.b[blockIdx.x] = s_rz;
+  }
+}
+
+// k_pcg_xpay and the next iteration's k_pcg_matvec_dot_sym64: the product
+// takes p = C r + b p of a row's neighbours from r, C and the old p, the
+// values that k_pcg_xpay would store, and the new p goes to a buffer of its
+// own (neighbours read the old one).  At max_iter the last iteration's x and
+// p are still formed, q is left.  G <= 2 kBlock partials of the update.
+template <int P, bool JAC>
+__global__ __launch_bounds__(kBlock) void k_pcg_step_sym64(
+    Sym64 A, double *__restrict__ x, const double *__restrict__ p, double *__restrict__ pnext,
+    double *__restrict__ q, const double *__restrict__ r, const double *__restrict__ C,
+    Partials prr, int G, Partials pq, SolveState *st, History h) {
+  __shared__ double lds[2][4], lds2[4];
+  const int chunk = sym64_chunk(A.n, blockIdx.x);
+  if (chunk < 0) return;
+  const int t = threadIdx.x, i = chunk * kBlock + t, row = min(i, A.n - 1);
+  double ra[2], rb[2];
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    ra[u] = prr.a[min(t + u * kBlock, G - 1)];
+    rb[u] = prr.b[min(t + u * kBlock, G - 1)];
+  }
+  const Scalars c = st->cur;
+  const double a = st->alpha, xi = x[row];
+  Sym64Loads<P> l;
+  sym64_load<P>(A, row, l);
+  double z[2 * P + 1], po[2 * P + 1];
+#pragma unroll
+  for (int k = 0; k < 2 * P + 1; k++) {
+    const int m = k < P ? max(row - A.off[k], 0) : k < 2 * P ? min(row + A.off[k - P], A.n - 1) : row;
+    z[k] = JAC ? elem(C, m) * elem(r, m) : elem(r, m);
+    po[k] = elem(p, m);
+  }
+  double r2 = 0.0, rz = 0.0;
+#pragma unroll
+  for (int u = 0; u < 2; u++) {
+    r2 = t + u * kBlock < G ? r2 + ra[u] : r2;
+    rz = t + u * kBlock < G ? rz + rb[u] : rz;
+  }
+  block_fold2(r2, rz, lds);
+  if (c.done) return;
+  const double rho = JAC ? rz : r2;
+  const double b = rho / c.rho;
+  const bool converged = end_iteration(st, c, r2, rho, b, h);
+  const bool goes_on = !converged && c.iteration + 1 < st->max_iter;
+  if (i < A.n) {
+    x[i] = xi + a * po[2 * P];
+    if (!converged) pnext[i] = z[2 * P] + b * po[2 * P];
+  }
+  if (!goes_on) return;
+  double pn[2 * P + 1];
+#pragma unroll
+  for (int k = 0; k < 2 * P + 1; k++) pn[k] = z[k] + b * po[k];
+  const double s = sym64_sum<P>(A, l, pn, pn + P, pn[2 * P], row);
+  double dot = 0.0;
+  if (i < A.n) {
+    q[i] = s;
+    dot = pn[2 * P] * s;
+  }
+  const double bp = block_fold(dot, lds2);
+  if (t == 0) pq.a[chunk] = bp;
 }
 
 }  // namespace
@@ -716,6 +906,34 @@ hipError_t pcg_matvec_dot_sym64(const Sym64 &A, const double *p, double *q, Part
   if (e == hipSuccess && pq2)
     hipLaunchKernelGGL(k_fold_groups, dim3(fold_groups(G)), dim3(kBlock), 0, s, pq.a, G, pq2);
   return e == hipSuccess ? hipGetLastError() : e;
+}
+
+hipError_t pcg_step_sym64(const Sym64 &A, double *x, const double *p, double *pnext, double *q,
+                          const double *r, const double *C, Partials pr, Partials pq,
+                          SolveState *st, History h, hipStream_t s) {
+  if (A.pairs < 1 || A.pairs > kSym64Pairs || ell_chunks(A.n) > kSmallChunks)
+    return hipErrorInvalidValue;
+  const dim3 grid(8 * ((ell_chunks(A.n) + 7) / 8));
+  auto launch = [&](auto k) {
+    hipLaunchKernelGGL(k, grid, dim3(kBlock), 0, s, A, x, p, pnext, q, r, C, pr, vec_grid(A.n), pq,
+                       st, h);
+  };
+  switch (A.pairs) {
+    case 1: C ? launch(k_pcg_step_sym64<1, true>) : launch(k_pcg_step_sym64<1, false>); break;
+    case 2: C ? launch(k_pcg_step_sym64<2, true>) : launch(k_pcg_step_sym64<2, false>); break;
+    default: C ? launch(k_pcg_step_sym64<3, true>) : launch(k_pcg_step_sym64<3, false>); break;
+  }
+  return hipGetLastError();
+}
+
+hipError_t pcg_update_small(int n, int G, double *r, const double *q, const double *C, Partials pq,
+                            Partials pr, SolveState *st, History h, hipStream_t s) {
+  if (ell_chunks(n) > kSmallChunks || G < 1 || G > kFoldDirect) return hipErrorInvalidValue;
+  auto launch = [&](auto k) {
+    hipLaunchKernelGGL(k, vgrid(n), dim3(kBlock), 0, s, n, G, r, q, C, pq.a, pr, st, h);
+  };
+  C ? launch(k_pcg_update_small<true>) : launch(k_pcg_update_small<false>);
+  return hipGetLastError();
 }
 
 hipError_t pcg_update(int n, int gpq, double *r, const double *q, const double *C, Partials pq,
