@@ -442,7 +442,7 @@ __device__ __forceinline__ double fold_two_levels(const double *__restrict__ par
   const double sum = 0.0 + (((lds[g][0] + lds[g][1]) + lds[g][2]) + lds[g][3]);
   const double w = wave_fold(lane < groups ? sum : 0.0);
   __syncthreads();
-  return __shfl(w, 0, 64) + 0.0;
+  return lane_first(w) + 0.0;
 }
 
 template <bool JAC>
