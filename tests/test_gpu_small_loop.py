@@ -81,3 +81,14 @@ def test_folded_partials(ctx, n):
     assert info["iterations"] == oit
     assert_bitwise(ctx.history("pq", oit), oh["pq"], "<p, q>")
     assert_bitwise(ctx.history("r2", oit + 1), oh["r2"], "<r, r>")
+
+
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 2047, 2049, 8191, 8192, 8193, 16385])
+def test_dot_hook(ctx, n):
+    """One block up to 16 partials (8,192 elements), two kernels above."""
+    rng = np.random.default_rng(n)
+    a, b = rng.standard_normal(n), rng.standard_normal(n)
+    ctx.set_size(n)
+    ctx.upload("P", a)
+    ctx.upload("Q", b)
+    assert_bitwise([ctx.dot("P", "Q")], [oracle.lib().orc_dot_tree(n, a, b)], "<p, q>")
