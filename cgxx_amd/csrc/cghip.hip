@@ -33,7 +33,7 @@ struct cghip_ctx {
 
   // CRS (MatrixDataCRS) + row blocks of the CSR-stream kernel
   bool has_crs = false;
-  int crs_nnz = 0, crs_nrb = 0, crs_short = 0;
+  int crs_nnz = 0, crs_nrb = 0, crs_short = 0, crs_longest = 0;
   int *crs_ptr = nullptr, *crs_index = nullptr, *crs_rb = nullptr;
   double *crs_value = nullptr;
 
@@ -344,6 +344,55 @@ hipError_t launch_matvec(cghip_ctx *c, const double *x, double *y) {
   return matvec_ell(ell_of(c), x, y, c->stream);
 }
 
+// Row blocks of a CRS matrix whose longest row is `longest` into rb: with
+// rows of up to kShortRow entries the greedy blocks are the kRowsMax-row
+// chunks, and the rows need not be walked.
+int row_blocks(int n, const int *ptr, int longest, std::vector<int> &rb) {
+  if (longest > kShortRow) {
+    rb.resize((size_t)n + 1);
+    return crs_rowblocks(n, ptr, rb.data());
+  }
+  const int nrb = ell_chunks(n);
+  rb.resize((size_t)nrb + 1);
+  for (int i = 0; i < nrb; i++) rb[i] = kRowsMax * i;
+  rb[nrb] = n;
+  return nrb;
+}
+
+// A copy on the device of `count` column indices, and whether all are in
+// range: check(copy, flag) raises the flag where one is not.  The copy is made
+// before anything of the context changes, so that a refused matrix leaves the
+// one before; without the memory for both at once it stays null and the
+// caller looks the indices over itself (*in_range false).  The check on the
+// device reads the copy in 20 us where a loop on the host took 5 ms (14.6
+// million entries).
+template <typename Check>
+int copy_columns(cghip_ctx *c, const int *index, int64_t count, int **copy, bool *in_range,
+                 Check check) {
+  *copy = nullptr;
+  *in_range = true;
+  if (count == 0) return CGHIP_OK;
+  *in_range = false;
+  int *d = nullptr;
+  if (hipMalloc((void **)&d, sizeof(int) * (size_t)count) != hipSuccess) {
+    (void)hipGetLastError();
+    return CGHIP_OK;
+  }
+  int *flag = reinterpret_cast<int *>(c->partial), bad = 1;
+  hipError_t e = hipMemcpy(d, index, sizeof(int) * (size_t)count, hipMemcpyHostToDevice);
+  if (e == hipSuccess) e = hipMemsetAsync(flag, 0, sizeof(int), c->stream);
+  if (e == hipSuccess) e = check(d, flag);
+  if (e == hipSuccess) e = hipMemcpyAsync(&bad, flag, sizeof(int), hipMemcpyDeviceToHost, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) {
+    (void)hipFree(d);
+    HIPCHK(c, e);
+  }
+  *copy = d;
+  *in_range = !bad;
+  return CGHIP_OK;
+}
+
 // Distinct off-diagonal offsets j - i of an uploaded matrix, ascending.
 struct Offsets {
   int count = -1;  // -1: more than kDiaMax, or columns out of order
@@ -525,21 +574,46 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
     return fail(c, CGHIP_ERR_ARG, "invalid CRS arguments (n=%d, nnz=%d)", n, nnz);
   if (ptr[0] != 0 || ptr[n] != nnz)
     return fail(c, CGHIP_ERR_ARG, "CRS ptr must start at 0 and end at nnz");
-  for (int i = 0; i < n; i++)
-    if (ptr[i + 1] < ptr[i]) return fail(c, CGHIP_ERR_ARG, "CRS ptr decreases at row %d", i);
-  for (int e = 0; e < nnz; e++)
-    if (index[e] < 0 || index[e] >= n)
-      return fail(c, CGHIP_ERR_ARG, "CRS column index %d out of range at entry %d", index[e], e);
-  if (c->n != n)
-    if (int rc = cghip_set_size(c, n)) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  int shortest = INT32_MAX, longest = 0;
+  for (int i = 0; i < n; i++) {
+    const int len = (int)((uint32_t)ptr[i + 1] - (uint32_t)ptr[i]);  // wraps only past a decrease
+    shortest = std::min(shortest, len);
+    longest = std::max(longest, len);
+  }
+  if (shortest < 0)
+    for (int i = 0; i < n; i++)
+      if (ptr[i + 1] < ptr[i]) return fail(c, CGHIP_ERR_ARG, "CRS ptr decreases at row %d", i);
+  HIPCHK(c, hipSetDevice(c->device));
+  int *new_index = nullptr;
+  bool in_range = true;
+  if (int rc = copy_columns(c, index, nnz, &new_index, &in_range, [&](const int *d, int *bad) {
+        return crs_columns(n, nnz, d, bad, c->stream);
+      }))
+    return rc;
+  if (!in_range)
+    for (int e = 0; e < nnz; e++)
+      if (index[e] < 0 || index[e] >= n) {
+        dfree(new_index);
+        return fail(c, CGHIP_ERR_ARG, "CRS column index %d out of range at entry %d", index[e], e);
+      }
+  auto begin = [&]() -> int {
+    if (c->n != n)
+      if (int rc = cghip_set_size(c, n)) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return CGHIP_OK;
+  };
+  if (int rc = begin()) {
+    dfree(new_index);
+    return rc;
+  }
   drop_graph(c);
   free_crs(c);
   free_fp32(c);
-  std::vector<int> rb((size_t)n + 1);
-  const int nrb = crs_rowblocks(n, ptr, rb.data());
+  std::vector<int> rb;
+  const int nrb = row_blocks(n, ptr, longest, rb);
+  c->crs_index = new_index;
   int rc = dalloc(c, &c->crs_ptr, (size_t)n + 1);
-  if (!rc) rc = dalloc(c, &c->crs_index, (size_t)nnz);
+  if (!rc && !c->crs_index) rc = dalloc(c, &c->crs_index, (size_t)nnz);
   if (!rc) rc = dalloc(c, &c->crs_value, (size_t)nnz);
   if (!rc) rc = dalloc(c, &c->crs_rb, (size_t)nrb + 1);
   if (rc) {
@@ -548,7 +622,8 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
   }
   HIPCHK(c, hipMemcpy(c->crs_ptr, ptr, sizeof(int) * ((size_t)n + 1), hipMemcpyHostToDevice));
   if (nnz > 0) {
-    HIPCHK(c, hipMemcpy(c->crs_index, index, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice));
+    if (!new_index)
+      HIPCHK(c, hipMemcpy(c->crs_index, index, sizeof(int) * (size_t)nnz, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->crs_value, value, sizeof(double) * (size_t)nnz, hipMemcpyHostToDevice));
   }
   HIPCHK(c, hipMemcpy(c->crs_rb, rb.data(), sizeof(int) * ((size_t)nrb + 1), hipMemcpyHostToDevice));
@@ -558,7 +633,8 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
   }
   c->crs_nnz = nnz;
   c->crs_nrb = nrb;
-  c->crs_short = crs_short_rows(n, ptr, nrb);
+  c->crs_longest = longest;
+  c->crs_short = longest <= kShortRow;
   Offsets o;
   rc = find_offsets(c, crs_of(c), &o);
   // rows of up to kShortRow entries: row blocks are 256-row chunks, so the
@@ -581,30 +657,76 @@ int cghip_upload_ell(cghip_ctx *c, int n, int width, const int32_t *length, cons
   if (n <= 0 || width < 0 || !length || (width > 0 && (!index || !data)))
     return fail(c, CGHIP_ERR_ARG, "invalid ELL arguments (n=%d, width=%d)", n, width);
   const int64_t slots = (int64_t)n * width;
+  HIPCHK(c, hipSetDevice(c->device));
+  int least = 0, most = 0;
   for (int i = 0; i < n; i++) {
-    if (length[i] < 0 || length[i] > width)
-      return fail(c, CGHIP_ERR_ARG, "ELL length[%d] = %d outside [0, %d]", i, length[i], width);
-    for (int j = 0; j < length[i]; j++) {
-      const int col = index[(int64_t)j * n + i];
-      if (col < 0 || col >= n)
-        return fail(c, CGHIP_ERR_ARG, "ELL column index %d out of range (row %d, slot %d)", col, i, j);
+    least = std::min(least, length[i]);
+    most = std::max(most, length[i]);
+  }
+  bool in_range = least >= 0 && most <= width;
+  int *new_length = nullptr, *new_index = nullptr;
+  auto drop = [&]() {
+    dfree(new_length);
+    dfree(new_index);
+  };
+  if (in_range && hipMalloc((void **)&new_length, sizeof(int) * (size_t)n) != hipSuccess) {
+    (void)hipGetLastError();
+    new_length = nullptr;
+    in_range = false;
+  }
+  if (in_range) {
+    int rc = CGHIP_OK;
+    const hipError_t e = hipMemcpy(new_length, length, sizeof(int) * (size_t)n, hipMemcpyHostToDevice);
+    if (e != hipSuccess) rc = fail(c, CGHIP_ERR_HIP, "copy of lengths: %s", hipGetErrorString(e));
+    if (!rc)
+      rc = copy_columns(c, index, slots, &new_index, &in_range, [&](const int *d, int *bad) {
+        return ell_columns(n, new_length, d, bad, c->stream);
+      });
+    if (rc) {
+      drop();
+      return rc;
     }
   }
-  if (c->n != n)
-    if (int rc = cghip_set_size(c, n)) return rc;
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  for (int i = 0; i < n && !in_range; i++) {
+    if (length[i] < 0 || length[i] > width) {
+      drop();
+      return fail(c, CGHIP_ERR_ARG, "ELL length[%d] = %d outside [0, %d]", i, length[i], width);
+    }
+    for (int j = 0; j < length[i]; j++) {
+      const int col = index[(int64_t)j * n + i];
+      if (col < 0 || col >= n) {
+        drop();
+        return fail(c, CGHIP_ERR_ARG, "ELL column index %d out of range (row %d, slot %d)", col, i, j);
+      }
+    }
+  }
+  auto begin = [&]() -> int {
+    if (c->n != n)
+      if (int rc = cghip_set_size(c, n)) return rc;
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return CGHIP_OK;
+  };
+  if (int rc = begin()) {
+    drop();
+    return rc;
+  }
   drop_graph(c);
   free_ell(c);
-  int rc = dalloc(c, &c->ell_length, (size_t)n);
-  if (!rc) rc = dalloc(c, &c->ell_index, (size_t)slots);
+  c->ell_length = new_length;
+  c->ell_index = new_index;
+  int rc = CGHIP_OK;
+  if (!c->ell_length) rc = dalloc(c, &c->ell_length, (size_t)n);
+  if (!rc && !c->ell_index) rc = dalloc(c, &c->ell_index, (size_t)slots);
   if (!rc) rc = dalloc(c, &c->ell_data, (size_t)slots);
   if (rc) {
     free_ell(c);
     return rc;
   }
-  HIPCHK(c, hipMemcpy(c->ell_length, length, sizeof(int) * (size_t)n, hipMemcpyHostToDevice));
+  if (!new_length)
+    HIPCHK(c, hipMemcpy(c->ell_length, length, sizeof(int) * (size_t)n, hipMemcpyHostToDevice));
   if (slots > 0) {
-    HIPCHK(c, hipMemcpy(c->ell_index, index, sizeof(int) * (size_t)slots, hipMemcpyHostToDevice));
+    if (!new_index)
+      HIPCHK(c, hipMemcpy(c->ell_index, index, sizeof(int) * (size_t)slots, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->ell_data, data, sizeof(double) * (size_t)slots, hipMemcpyHostToDevice));
   }
   if (int e = ensure_pq1(c, std::max(ell_chunks(n), 1))) {
@@ -982,6 +1104,31 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
 
 // ---- mixed precision -----------------------------------------------------
 
+namespace {
+
+// The scaled operator in CRS, for matrices that neither DIA nor ELL holds:
+// the row pointer is ptr[i] - i, the row blocks those of the shorter rows.
+int scaled_crs(cghip_ctx *c) {
+  const int n = c->n;
+  std::vector<int> ptr((size_t)n + 1), rb;
+  HIPCHK(c, hipMemcpy(ptr.data(), c->crs_ptr, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost));
+  for (int i = 0; i <= n; i++) ptr[i] -= i;
+  c->short_nd = c->crs_longest - 1 <= kShortRow;
+  c->nrb_nd = row_blocks(n, ptr.data(), c->crs_longest - 1, rb);
+  int rc = dalloc(c, &c->ptr_nd, (size_t)n + 1);
+  if (!rc) rc = dalloc(c, &c->index_nd, (size_t)c->nnz_nd);
+  if (!rc) rc = dalloc(c, &c->value_nd, (size_t)c->nnz_nd);
+  if (!rc) rc = dalloc(c, &c->rb_nd, (size_t)c->nrb_nd + 1);
+  if (rc) return rc;
+  HIPCHK(c, hipMemcpy(c->ptr_nd, ptr.data(), sizeof(int) * ((size_t)n + 1), hipMemcpyHostToDevice));
+  HIPCHK(c, hipMemcpy(c->rb_nd, rb.data(), sizeof(int) * ((size_t)c->nrb_nd + 1),
+                      hipMemcpyHostToDevice));
+  HIPCHK(c, scaled_copy(crs_of(c), c->scale64, c->index_nd, c->value_nd, c->stream));
+  return CGHIP_OK;
+}
+
+}  // namespace
+
 int cghip_prepare_fp32(cghip_ctx *c) {
   if (!c) return CGHIP_ERR_ARG;
   if (!c->has_crs) return fail(c, CGHIP_ERR_STATE, "mixed precision needs a CRS matrix");
@@ -1014,29 +1161,9 @@ int cghip_prepare_fp32(cghip_ctx *c) {
   HIPCHK(c, hipMemcpyAsync(&bad, d_bad, sizeof(int), hipMemcpyDeviceToHost, c->stream));
   if (int r = sync(c)) return r;
   if (!bad) {
-    // row i keeps ptr[i+1] - ptr[i] - 1 entries: the off-diagonal row
-    // pointer is ptr[i] - i
-    std::vector<int> ptr(n + 1);
-    HIPCHK(c, hipMemcpy(ptr.data(), c->crs_ptr, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
-    for (int i = 0; i <= n; i++) ptr[i] -= i;
-    c->nnz_nd = ptr[n];
-    std::vector<int> starts(n + 1);
-    c->nrb_nd = crs_rowblocks(n, ptr.data(), starts.data());
-    c->short_nd = crs_short_rows(n, ptr.data(), c->nrb_nd);
-    rc = dalloc(c, &c->ptr_nd, (size_t)n + 1);
-    if (!rc) rc = dalloc(c, &c->index_nd, (size_t)c->nnz_nd);
-    if (!rc) rc = dalloc(c, &c->value_nd, (size_t)c->nnz_nd);
-    if (!rc) rc = dalloc(c, &c->rb_nd, (size_t)c->nrb_nd + 1);
-    if (rc) {
-      free_fp32(c);
-      return rc;
-    }
-    HIPCHK(c, hipMemcpy(c->ptr_nd, ptr.data(), sizeof(int) * (n + 1), hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(c->rb_nd, starts.data(), sizeof(int) * (c->nrb_nd + 1),
-                        hipMemcpyHostToDevice));
-    HIPCHK(c, scaled_copy(crs_of(c), c->scale64, c->index_nd, c->value_nd, c->stream));
-    int w = 0;
-    for (int i = 0; i < n; i++) w = std::max(w, ptr[i + 1] - ptr[i]);
+    // row i keeps ptr[i+1] - ptr[i] - 1 entries
+    c->nnz_nd = c->crs_nnz - n;
+    const int w = c->crs_longest - 1;
     if (c->dia_ndiag > 0 && dia_pays(c->dia_ndiag, n, c->nnz_nd)) {
       // a tile past the last stream: rows of a quad past the last row
       const size_t slots = (size_t)c->dia_ndiag * (size_t)n + (c->pad32 ? kQuadTile : 0);
@@ -1091,6 +1218,11 @@ int cghip_prepare_fp32(cghip_ctx *c) {
       c->ell_nd = true;
       c->ell_w_nd = w;
     }
+    if (!c->dia_nd && !c->ell_nd)
+      if (int r = scaled_crs(c)) {
+        free_fp32(c);
+        return r;
+      }
     if (int r = sync(c)) return r;
     c->has_scaled = true;
   }

@@ -163,9 +163,6 @@ inline bool sym64_fits(int64_t n) { return 8 * n <= (1ll << 32); }
 // kNnzCap nonzeros, except that a block always takes its first row (a row
 // longer than kNnzCap is then streamed through LDS in chunks).
 int crs_rowblocks(int n, const int *ptr, int *starts);
-// 1 if every row of ptr has at most kShortRow entries and the row blocks
-// from crs_rowblocks are the full kRowsMax-row blocks that implies.
-int crs_short_rows(int n, const int *ptr, int nrb);
 
 // Message returned by cghip_last_error(NULL) (errors without a context).
 void set_global_error(const char *msg);
@@ -204,6 +201,11 @@ hipError_t pcg_matvec_dot_ell(const Ell<double> &A, const double *p, double *q, 
 hipError_t matvec_sym64(const Sym64 &A, const double *x, double *y, hipStream_t s);
 hipError_t pcg_matvec_dot_sym64(const Sym64 &A, const double *p, double *q, Partials pq,
                                 double *pq2, SolveState *st, hipStream_t s);
+// bad[0] = 1 (0 beforehand) if one of nnz column indices, or of the live ones
+// of an ELL matrix (the first length[i] of row i, column-major), lies outside
+// [0, n).
+hipError_t crs_columns(int n, int nnz, const int *index, int *bad, hipStream_t s);
+hipError_t ell_columns(int n, const int *length, const int *index, int *bad, hipStream_t s);
 // Diagonals of an uploaded matrix.  matrix_offsets: found[1 .. kDiaMax] the
 // distinct off-diagonal offsets in no order (INT32_MIN: none), found[0] the
 // flags kOffsetsIrregular (a row's columns do not ascend, or more than

@@ -82,6 +82,27 @@ __global__ __launch_bounds__(kBlock) void k_offsets(M A, int *__restrict__ found
     atomicOr(found, kOffsetsIrregular);
 }
 
+// Column indices against [0, n), one pass at the rate of a copy.
+__global__ __launch_bounds__(kBlock) void k_crs_columns(int n, int64_t nnz,
+                                                        const int *__restrict__ index,
+                                                        int *__restrict__ bad) {
+  const int64_t T = (int64_t)gridDim.x * kBlock;
+  bool out = false;
+  for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < nnz; e += T)
+    out |= (uint32_t)index[e] >= (uint32_t)n;
+  if (out) bad[0] = 1;
+}
+
+__global__ __launch_bounds__(kBlock) void k_ell_columns(int n, const int *__restrict__ length,
+                                                        const int *__restrict__ index,
+                                                        int *__restrict__ bad) {
+  const int64_t T = (int64_t)gridDim.x * kBlock;
+  bool out = false;
+  for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n; i += T)
+    for (int j = 0; j < length[i]; j++) out |= (uint32_t)index[(int64_t)j * n + i] >= (uint32_t)n;
+  if (out) bad[0] = 1;
+}
+
 // The row's diagonal and upper entries, absent where it has none.
 template <typename Row, typename M>
 __global__ __launch_bounds__(kBlock) void k_sym64_build(M A, Sym64 S, double *__restrict__ diag,
@@ -171,6 +192,15 @@ hipError_t build_t(const M &A, const Sym64 &S, double *diag, double *up, int *fo
 
 }  // namespace
 
+hipError_t crs_columns(int n, int nnz, const int *index, int *bad, hipStream_t s) {
+  hipLaunchKernelGGL(k_crs_columns, dim3(setup_grid(nnz)), dim3(kBlock), 0, s, n, (int64_t)nnz, index,
+                     bad);
+  return hipGetLastError();
+}
+hipError_t ell_columns(int n, const int *length, const int *index, int *bad, hipStream_t s) {
+  hipLaunchKernelGGL(k_ell_columns, dim3(setup_grid(n)), dim3(kBlock), 0, s, n, length, index, bad);
+  return hipGetLastError();
+}
 hipError_t matrix_offsets(const Crs<double> &A, int *found, hipStream_t s) {
   return offsets_t<CrsRow>(A, found, s);
 }
