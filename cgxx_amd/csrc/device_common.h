@@ -6,6 +6,7 @@
 #include "cghip_kernels.h"
 
 #include <type_traits>
+#include <utility>
 
 #pragma clang fp contract(off)
 
@@ -99,22 +100,23 @@ __device__ inline double thread_partials(const double *partial, int G) {
   return s;
 }
 
-// The same for two arrays (ga, gb >= 1 partials) with both arrays' loads in
-// flight together.
+// The same for two arrays (ga, gb >= 1 partials) with both arrays' loads, B at
+// a time, in flight together.
+template <int B = 8>
 __device__ inline void thread_partials2(const double *a, int ga, const double *b, int gb,
                                         double &sa, double &sb) {
   sa = 0.0;
   sb = 0.0;
   const int g = max(ga, gb);
-  for (int i = threadIdx.x; i < g; i += 8 * kBlock) {
-    double va[8], vb[8];
+  for (int i = threadIdx.x; i < g; i += B * kBlock) {
+    double va[B], vb[B];
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < B; u++) {
       va[u] = a[min(i + u * kBlock, ga - 1)];
       vb[u] = b[min(i + u * kBlock, gb - 1)];
     }
 #pragma unroll
-    for (int u = 0; u < 8; u++) {
+    for (int u = 0; u < B; u++) {
       sa = i + u * kBlock < ga ? sa + va[u] : sa;
       sb = i + u * kBlock < gb ? sb + vb[u] : sb;
     }
@@ -129,10 +131,11 @@ __device__ inline double fold_partials(const double *partial, int G, double *lds
 }
 
 // Two such folds, their loads in flight together.
+template <int B = 8>
 __device__ inline void fold_partials2(const double *a, int ga, const double *b, int gb,
                                       double *lds, double &ra, double &rb) {
   double sa, sb;
-  thread_partials2(a, ga, b, gb, sa, sb);
+  thread_partials2<B>(a, ga, b, gb, sa, sb);
   ra = block_fold(sa, lds);
   rb = block_fold(sb, lds);
 }
@@ -745,6 +748,55 @@ struct Quads {
 
 __device__ inline const float4 *v4(const float *p) { return reinterpret_cast<const float4 *>(p); }
 __device__ inline float4 *v4(float *p) { return reinterpret_cast<float4 *>(p); }
+
+// A thread's whole groups q, q + T, ... below full, U in flight: load(i) is
+// group i's operands, use(i, operands) runs for each in ascending order.  A
+// place past the last group loads the thread's own first one again (not the
+// vector's last, which every wave would then fetch at once) and is dropped,
+// so the groups of a short vector are loads of whole groups too: a loop over
+// single elements for the groups that do not fill U places took 2 to 4 us more
+// per FP32 kernel at 128^3, where no thread has U of them (mixed Jacobi
+// iteration 38.5 -> 32.4 us).  The first U loads go out when it is made,
+// before the kernel waits for its scalars (FP64 iteration at 128^3 55.8 ->
+// 53.8 us, at 256^3 426 -> 418).
+template <int U, typename L>
+struct Trips {
+  typedef decltype(std::declval<L>()((int64_t)0)) V;
+  V v[U];
+  int64_t q, T, full;
+  L load;
+  __device__ __forceinline__ Trips(int64_t q0, int64_t stride, int64_t count, L l)
+      : q(q0), T(stride), full(count), load(l) {
+    if (full > 0) fetch();
+  }
+  __device__ __forceinline__ void fetch() {
+    const int64_t own = q < full ? q : full - 1;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int64_t i = q + u * T;
+      v[u] = load(i < full ? i : own);
+    }
+  }
+  template <typename Use>
+  __device__ __forceinline__ void run(Use use) {
+    while (q < full) {
+#pragma unroll
+      for (int u = 0; u < U; u++)
+        if (q + u * T < full) use(q + u * T, v[u]);
+      q += U * T;
+      if (q < full) fetch();
+    }
+  }
+};
+template <int U, typename G, typename L>
+__device__ __forceinline__ Trips<U, L> trips(const G &g, L load) {
+  return Trips<U, L>(g.q, g.T, g.full, load);
+}
+// Whether this thread owns the last, partial group.
+template <typename G>
+__device__ inline bool owns_rest(const G &g, int64_t groups) {
+  return groups > g.full && g.full % g.T == g.q;
+}
 
 }  // namespace dev
 }  // namespace cghip

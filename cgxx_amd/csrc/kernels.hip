@@ -219,77 +219,48 @@ __global__ __launch_bounds__(kBlock) void k_fold_groups(const double *__restrict
 // pairs gid, gid + T, ... in order, element 2q before 2q+1.  The last pair
 // of an odd-length vector holds one element.
 
+struct Pairs2 {
+  double2 a, b;
+};
+struct Pairs3 {
+  double2 a, b, c;
+};
+struct Pairs4 {
+  double2 a, b, c, d;
+};
+
 __global__ __launch_bounds__(kBlock) void k_axpy(int n, double a, const double *__restrict__ x,
                                                  double *__restrict__ y) {
-  Pairs P(n);
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 xv[kUnroll], yv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      xv[u] = v2(x)[P.q + u * P.T];
-      yv[u] = v2(y)[P.q + u * P.T];
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      yv[u].x = yv[u].x + a * xv[u].x;
-      yv[u].y = yv[u].y + a * xv[u].y;
-      v2(y)[P.q + u * P.T] = yv[u];
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    const int64_t e = 2 * P.q;
-    y[e] = y[e] + a * x[e];
-    if (e + 1 < n) y[e + 1] = y[e + 1] + a * x[e + 1];
-  }
+  const Pairs P(n);
+  trips<kUnroll>(P, [=](int64_t j) { return Pairs2{v2(x)[j], v2(y)[j]}; })
+      .run([&](int64_t j, Pairs2 &v) {
+        v.b.x = v.b.x + a * v.a.x;
+        v.b.y = v.b.y + a * v.a.y;
+        v2(y)[j] = v.b;
+      });
+  if (owns_rest(P, P.npair)) y[n - 1] = y[n - 1] + a * x[n - 1];
 }
 
 __global__ __launch_bounds__(kBlock) void k_xpay(int n, const double *__restrict__ x, double a,
                                                  double *__restrict__ y) {
-  Pairs P(n);
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 xv[kUnroll], yv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      xv[u] = v2(x)[P.q + u * P.T];
-      yv[u] = v2(y)[P.q + u * P.T];
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      yv[u].x = xv[u].x + a * yv[u].x;
-      yv[u].y = xv[u].y + a * yv[u].y;
-      v2(y)[P.q + u * P.T] = yv[u];
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    const int64_t e = 2 * P.q;
-    y[e] = x[e] + a * y[e];
-    if (e + 1 < n) y[e + 1] = x[e + 1] + a * y[e + 1];
-  }
+  const Pairs P(n);
+  trips<kUnroll>(P, [=](int64_t j) { return Pairs2{v2(x)[j], v2(y)[j]}; })
+      .run([&](int64_t j, Pairs2 &v) {
+        v.b.x = v.a.x + a * v.b.x;
+        v.b.y = v.a.y + a * v.b.y;
+        v2(y)[j] = v.b;
+      });
+  if (owns_rest(P, P.npair)) y[n - 1] = x[n - 1] + a * y[n - 1];
 }
 
 __global__ __launch_bounds__(kBlock) void k_jacobi(int n, const double *__restrict__ C,
                                                    const double *__restrict__ x, double *__restrict__ y) {
-  Pairs P(n);
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 cv[kUnroll], xv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      cv[u] = v2(C)[P.q + u * P.T];
-      xv[u] = v2(x)[P.q + u * P.T];
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      double2 yv;
-      yv.x = cv[u].x * xv[u].x;
-      yv.y = cv[u].y * xv[u].y;
-      v2(y)[P.q + u * P.T] = yv;
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    const int64_t e = 2 * P.q;
-    y[e] = C[e] * x[e];
-    if (e + 1 < n) y[e + 1] = C[e + 1] * x[e + 1];
-  }
+  const Pairs P(n);
+  trips<kUnroll>(P, [=](int64_t j) { return Pairs2{v2(C)[j], v2(x)[j]}; })
+      .run([&](int64_t j, Pairs2 &v) {
+        v2(y)[j] = make_double2(v.a.x * v.b.x, v.a.y * v.b.y);
+      });
+  if (owns_rest(P, P.npair)) y[n - 1] = C[n - 1] * x[n - 1];
 }
 
 __global__ __launch_bounds__(kBlock) void k_fill(int n, double v, double *__restrict__ y) {
@@ -300,26 +271,14 @@ __global__ __launch_bounds__(kBlock) void k_fill(int n, double v, double *__rest
 __global__ __launch_bounds__(kBlock) void k_dot_partials(int n, const double *__restrict__ a,
                                                          const double *__restrict__ b, Partials pa) {
   __shared__ double lds[4];
-  Pairs P(n);
+  const Pairs P(n);
   double s = 0.0;
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 av[kUnroll], bv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      av[u] = v2(a)[P.q + u * P.T];
-      bv[u] = v2(b)[P.q + u * P.T];
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      s += av[u].x * bv[u].x;
-      s += av[u].y * bv[u].y;
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    const int64_t e = 2 * P.q;
-    s += a[e] * b[e];
-    if (e + 1 < n) s += a[e + 1] * b[e + 1];
-  }
+  trips<kUnroll>(P, [=](int64_t j) { return Pairs2{v2(a)[j], v2(b)[j]}; })
+      .run([&](int64_t, Pairs2 &v) {
+        s += v.a.x * v.b.x;
+        s += v.a.y * v.b.y;
+      });
+  if (owns_rest(P, P.npair)) s += a[n - 1] * b[n - 1];
   const double bp = block_fold(s, lds);
   if (threadIdx.x == 0) pa.a[blockIdx.x] = bp;
 }
@@ -416,18 +375,24 @@ __global__ __launch_bounds__(kBlock) void k_pcg_init(int n, const double *__rest
                                                      double *__restrict__ r, double *__restrict__ p,
                                                      const double *__restrict__ C, Partials pa) {
   __shared__ double lds[4];
-  Pairs P(n);
+  const Pairs P(n);
   double s_rr = 0.0, s_pr = 0.0;
-  for (; P.q < P.npair; P.q += P.T) {
-    for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++) {
-      const double ri = k[e] + (-1.0) * r[e];
-      r[e] = ri;
-      const double pi = JAC ? C[e] * ri : ri;
-      p[e] = pi;
-      s_rr += ri * ri;
-      s_pr += pi * ri;
-    }
-  }
+  auto init = [&](double ke, double ce, double &re, double &pe) {
+    re = ke + (-1.0) * re;
+    pe = JAC ? ce * re : re;
+    s_rr += re * re;
+    s_pr += pe * re;
+  };
+  trips<kUnroll>(P, [=](int64_t j) {
+    return Pairs3{v2(k)[j], v2(r)[j], JAC ? v2(C)[j] : make_double2(0.0, 0.0)};
+  }).run([&](int64_t j, Pairs3 &v) {
+    double2 pv;
+    init(v.a.x, v.c.x, v.b.x, pv.x);
+    init(v.a.y, v.c.y, v.b.y, pv.y);
+    v2(r)[j] = v.b;
+    v2(p)[j] = pv;
+  });
+  if (owns_rest(P, P.npair)) init(k[n - 1], JAC ? C[n - 1] : 0.0, r[n - 1], p[n - 1]);
   const double b0 = block_fold(s_rr, lds);
   const double b1 = block_fold(s_pr, lds);
   if (threadIdx.x == 0) {
@@ -503,6 +468,11 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     const double *__restrict__ C, Partials ppq, Partials prr, SolveState *st, History h) {
   __shared__ double lds[4];
   __shared__ double lds2[kFoldDirect / kBlock][4];
+  const Pairs P(n);
+  auto pairs = trips<2>(P, [=](int64_t j) {
+    return Pairs3{v2(r)[j], NT ? v2_stream(q, j) : v2(q)[j],
+                  !JAC ? make_double2(0.0, 0.0) : NT ? v2_stream(C, j) : v2(C)[j]};
+  });
   const Scalars c = st->cur;
   if (c.done) return;
   const double pq =
@@ -514,31 +484,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     if (h.alpha && c.iteration < h.cap) h.alpha[c.iteration] = a;
   }
   const double na = -a;
-  Pairs P(n);
   double s_rr = 0.0, s_rz = 0.0;
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 rv[kUnroll], qv[kUnroll], cv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      const int64_t j = P.q + u * P.T;
-      rv[u] = v2(r)[j];
-      qv[u] = NT ? v2_stream(q, j) : v2(q)[j];
-      if (JAC) cv[u] = NT ? v2_stream(C, j) : v2(C)[j];
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      const int64_t j = P.q + u * P.T;
-      update_elem<JAC>(rv[u].x, qv[u].x, JAC ? cv[u].x : 0.0, na, s_rr, s_rz);
-      update_elem<JAC>(rv[u].y, qv[u].y, JAC ? cv[u].y : 0.0, na, s_rr, s_rz);
-      v2(r)[j] = rv[u];
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++) {
-      double re = r[e];
-      update_elem<JAC>(re, q[e], JAC ? C[e] : 0.0, na, s_rr, s_rz);
-      r[e] = re;
-    }
+  pairs.run([&](int64_t j, Pairs3 &v) {
+    update_elem<JAC>(v.a.x, v.b.x, v.c.x, na, s_rr, s_rz);
+    update_elem<JAC>(v.a.y, v.b.y, v.c.y, na, s_rr, s_rz);
+    v2(r)[j] = v.a;
+  });
+  if (owns_rest(P, P.npair)) {
+    double re = r[n - 1];
+    update_elem<JAC>(re, q[n - 1], JAC ? C[n - 1] : 0.0, na, s_rr, s_rz);
+    r[n - 1] = re;
   }
   const double b0 = block_fold(s_rr, lds);
   const double b1 = block_fold(s_rz, lds);
@@ -585,11 +540,16 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
     int n, double *__restrict__ x, double *__restrict__ p, const double *__restrict__ r,
     const double *__restrict__ C, Partials prr, SolveState *st, History h) {
   __shared__ double lds[4];
+  const Pairs P(n);
+  auto pairs = trips<2>(P, [=](int64_t j) {
+    return Pairs4{NT ? v2_stream(x, j) : v2(x)[j], v2(p)[j], NT ? v2_stream(r, j) : v2(r)[j],
+                  !JAC ? make_double2(0.0, 0.0) : NT ? v2_stream(C, j) : v2(C)[j]};
+  });
   const Scalars c = st->cur;
   if (c.done) return;
   const int G = gridDim.x;  // the update kernel ran on the same grid
   double r2, rz;
-  fold_partials2(prr.a, G, prr.b, G, lds, r2, rz);
+  fold_partials2<4>(prr.a, G, prr.b, G, lds, r2, rz);
   const double rho = JAC ? rz : r2;
   const double b = rho / c.rho;
   const double a = st->alpha;
@@ -597,46 +557,29 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
   // x += a p always; p = z + b p unless the loop stops here.  Four streams
   // per element: unrolled twice to stay within 64 VGPRs.  x, r and C are
   // streamed non-temporally: only p stays cached for the next SpMV.
-  constexpr int U = 2;
-  Pairs P(n);
   if (converged) {
-    for (; P.q < P.npair; P.q += P.T)
-      for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++) x[e] = x[e] + a * p[e];
+    for (int64_t g = P.q; g < P.npair; g += P.T)
+      for (int64_t e = 2 * g; e < 2 * g + 2 && e < n; e++) x[e] = x[e] + a * p[e];
     return;
   }
-  for (; P.q + (U - 1) * P.T < P.full; P.q += U * P.T) {
-    double2 xv[U], pv[U], rv[U], cv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int64_t j = P.q + u * P.T;
-      xv[u] = NT ? v2_stream(x, j) : v2(x)[j];
-      pv[u] = v2(p)[j];
-      rv[u] = NT ? v2_stream(r, j) : v2(r)[j];
-      if (JAC) cv[u] = NT ? v2_stream(C, j) : v2(C)[j];
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int64_t j = P.q + u * P.T;
-      xv[u].x = xv[u].x + a * pv[u].x;
-      xv[u].y = xv[u].y + a * pv[u].y;
-      const double zx = JAC ? cv[u].x * rv[u].x : rv[u].x;
-      const double zy = JAC ? cv[u].y * rv[u].y : rv[u].y;
-      pv[u].x = zx + b * pv[u].x;
-      pv[u].y = zy + b * pv[u].y;
-      if (NT)
-        v2_store_stream(x, j, xv[u]);
-      else
-        v2(x)[j] = xv[u];
-      v2(p)[j] = pv[u];
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++) {
-      const double pe = p[e];
-      x[e] = x[e] + a * pe;
-      const double ze = JAC ? C[e] * r[e] : r[e];
-      p[e] = ze + b * pe;
-    }
+  pairs.run([&](int64_t j, Pairs4 &v) {
+    v.a.x = v.a.x + a * v.b.x;
+    v.a.y = v.a.y + a * v.b.y;
+    const double zx = JAC ? v.d.x * v.c.x : v.c.x;
+    const double zy = JAC ? v.d.y * v.c.y : v.c.y;
+    v.b.x = zx + b * v.b.x;
+    v.b.y = zy + b * v.b.y;
+    if (NT)
+      v2_store_stream(x, j, v.a);
+    else
+      v2(x)[j] = v.a;
+    v2(p)[j] = v.b;
+  });
+  if (owns_rest(P, P.npair)) {
+    const double pe = p[n - 1];
+    x[n - 1] = x[n - 1] + a * pe;
+    const double ze = JAC ? C[n - 1] * r[n - 1] : r[n - 1];
+    p[n - 1] = ze + b * pe;
   }
 }
 

@@ -295,30 +295,23 @@ __device__ inline double op32_rows(const Op32 &A, const float *__restrict__ x, f
 __global__ __launch_bounds__(kBlock) void k_mp_accum(int n, double *__restrict__ x64,
                                                      const float *__restrict__ y32,
                                                      const double *__restrict__ scale) {
-  constexpr int U = 2;
-  Pairs P(n);
+  struct V {
+    double2 x, s;
+    float2 y;
+  };
+  const Pairs P(n);
   const float2 *y2 = reinterpret_cast<const float2 *>(y32);
-  for (; P.q + (U - 1) * P.T < P.full; P.q += U * P.T) {
-    double2 xv[U], sv[U];
-    float2 yv[U];
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int64_t j = P.q + u * P.T;
-      xv[u] = v2(x64)[j];
-      yv[u] = y2[j];
-      sv[u] = scale ? v2_stream(scale, j) : make_double2(0.0, 0.0);
-    }
-#pragma unroll
-    for (int u = 0; u < U; u++) {
-      const int64_t j = P.q + u * P.T;
-      xv[u].x = xv[u].x + (scale ? sv[u].x * (double)yv[u].x : (double)yv[u].x);
-      xv[u].y = xv[u].y + (scale ? sv[u].y * (double)yv[u].y : (double)yv[u].y);
-      v2(x64)[j] = xv[u];
-    }
+  trips<2>(P, [=](int64_t j) {
+    return V{v2(x64)[j], scale ? v2_stream(scale, j) : make_double2(0.0, 0.0), y2[j]};
+  }).run([&](int64_t j, V &v) {
+    v.x.x = v.x.x + (scale ? v.s.x * (double)v.y.x : (double)v.y.x);
+    v.x.y = v.x.y + (scale ? v.s.y * (double)v.y.y : (double)v.y.y);
+    v2(x64)[j] = v.x;
+  });
+  if (owns_rest(P, P.npair)) {
+    const int64_t e = 2 * P.full;
+    x64[e] = x64[e] + (scale ? scale[e] * (double)y32[e] : (double)y32[e]);
   }
-  for (; P.q < P.npair; P.q += P.T)
-    for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++)
-      x64[e] = x64[e] + (scale ? scale[e] * (double)y32[e] : (double)y32[e]);
 }
 
 // r64 = k - q64 and the partials of ||r64||^2 (pairs order: a thread's
@@ -327,30 +320,23 @@ __global__ __launch_bounds__(kBlock) void k_mp_residual(int n, const double *__r
                                                         const double *__restrict__ q,
                                                         double *__restrict__ r, Partials pa) {
   __shared__ double lds[4];
-  Pairs P(n);
+  struct V {
+    double2 k, q;
+  };
+  const Pairs P(n);
   double s = 0.0;
-  for (; P.q + (kUnroll - 1) * P.T < P.full; P.q += kUnroll * P.T) {
-    double2 kv[kUnroll], qv[kUnroll];
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      const int64_t j = P.q + u * P.T;
-      kv[u] = v2_stream(k, j);
-      qv[u] = v2_stream(q, j);
-    }
-#pragma unroll
-    for (int u = 0; u < kUnroll; u++) {
-      const double r0 = kv[u].x - qv[u].x, r1 = kv[u].y - qv[u].y;
-      v2(r)[P.q + u * P.T] = make_double2(r0, r1);
-      s += r0 * r0;
-      s += r1 * r1;
-    }
-  }
-  for (; P.q < P.npair; P.q += P.T) {
-    for (int64_t e = 2 * P.q; e < 2 * P.q + 2 && e < n; e++) {
-      const double ri = k[e] - q[e];
-      r[e] = ri;
-      s += ri * ri;
-    }
+  trips<kUnroll>(P, [=](int64_t j) { return V{v2_stream(k, j), v2_stream(q, j)}; })
+      .run([&](int64_t j, V &v) {
+        const double r0 = v.k.x - v.q.x, r1 = v.k.y - v.q.y;
+        v2(r)[j] = make_double2(r0, r1);
+        s += r0 * r0;
+        s += r1 * r1;
+      });
+  if (owns_rest(P, P.npair)) {
+    const int64_t e = 2 * P.full;
+    const double ri = k[e] - q[e];
+    r[e] = ri;
+    s += ri * ri;
   }
   const double bp = block_fold(s, lds);
   if (threadIdx.x == 0) pa.a[blockIdx.x] = bp;
@@ -370,47 +356,35 @@ __global__ __launch_bounds__(kBlock) void k_mp_restart(int n, const double *__re
                                                        float *__restrict__ p32, int first,
                                                        Partials pb) {
   __shared__ double lds[4];
-  Quads Q(n);
+  struct V {
+    double2 ra, rb, sa, sb;
+  };
+  const Quads Q(n);
   double s_rr = 0.0;
-  for (; Q.q + (kQuadUnroll - 1) * Q.T < Q.full; Q.q += kQuadUnroll * Q.T) {
-    double2 ra[kQuadUnroll], rb[kQuadUnroll], sa[kQuadUnroll], sb[kQuadUnroll];
-#pragma unroll
-    for (int u = 0; u < kQuadUnroll; u++) {
-      const int64_t j = Q.q + u * Q.T;
-      ra[u] = v2_stream(r64, 2 * j);
-      rb[u] = v2_stream(r64, 2 * j + 1);
-      if (scale) {
-        sa[u] = v2_stream(scale, 2 * j);
-        sb[u] = v2_stream(scale, 2 * j + 1);
-      } else {
-        sa[u] = sb[u] = make_double2(0.0, 0.0);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < kQuadUnroll; u++) {
-      const int64_t j = Q.q + u * Q.T;
-      const float4 rv = make_float4(restart_value(ra[u].x, scale, sa[u].x),
-                                    restart_value(ra[u].y, scale, sa[u].y),
-                                    restart_value(rb[u].x, scale, sb[u].x),
-                                    restart_value(rb[u].y, scale, sb[u].y));
-      v4(r32)[j] = rv;
-      v4(y32)[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-      if (first) v4(p32)[j] = rv;
-      s_rr += (double)rv.x * (double)rv.x;
-      s_rr += (double)rv.y * (double)rv.y;
-      s_rr += (double)rv.z * (double)rv.z;
-      s_rr += (double)rv.w * (double)rv.w;
-    }
-  }
-  for (; Q.q < Q.nquad; Q.q += Q.T) {
-    for (int64_t e = 4 * Q.q; e < 4 * Q.q + 4 && e < n; e++) {
+  trips<kQuadUnroll>(Q, [=](int64_t j) {
+    const double2 zero = make_double2(0.0, 0.0);
+    return V{v2_stream(r64, 2 * j), v2_stream(r64, 2 * j + 1),
+             scale ? v2_stream(scale, 2 * j) : zero, scale ? v2_stream(scale, 2 * j + 1) : zero};
+  }).run([&](int64_t j, V &v) {
+    const float4 rv = make_float4(
+        restart_value(v.ra.x, scale, v.sa.x), restart_value(v.ra.y, scale, v.sa.y),
+        restart_value(v.rb.x, scale, v.sb.x), restart_value(v.rb.y, scale, v.sb.y));
+    v4(r32)[j] = rv;
+    v4(y32)[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (first) v4(p32)[j] = rv;
+    s_rr += (double)rv.x * (double)rv.x;
+    s_rr += (double)rv.y * (double)rv.y;
+    s_rr += (double)rv.z * (double)rv.z;
+    s_rr += (double)rv.w * (double)rv.w;
+  });
+  if (owns_rest(Q, Q.nquad))
+    for (int64_t e = 4 * Q.full; e < n; e++) {
       const float r = restart_value(r64[e], scale, scale ? scale[e] : 0.0);
       r32[e] = r;
       y32[e] = 0.0f;
       if (first) p32[e] = r;
       s_rr += (double)r * (double)r;
     }
-  }
   const double b0 = block_fold(s_rr, lds);
   if (threadIdx.x == 0) pb.a[blockIdx.x] = b0;
 }
@@ -487,12 +461,21 @@ __device__ inline void mp_update_elem(float &r, float q, float na, double &s_rr)
   s_rr += (double)r * (double)r;
 }
 
+struct Quads2 {
+  float4 a, b;
+};
+struct Quads3 {
+  float4 a, b, c;
+};
+
 // alpha = rho / <p,q> (into st->alpha32 for the p update, which also does
 // y32 += alpha p32); r32 -= alpha q32; partials of <r,r>.
 __global__ __launch_bounds__(kBlock) void k_mp_update(int n, int gpq, float *__restrict__ r,
                                                       const float *__restrict__ q, Partials ppq,
                                                       Partials prr, MixedState *st, History h) {
   __shared__ double lds[4];
+  const Quads Q(n);
+  auto quads = trips<kQuadUnroll>(Q, [=](int64_t j) { return Quads2{v4(r)[j], v4(q)[j]}; });
   const MixedScalars c = st->cur;
   if (c.done) return;
   const double pq = fold_partials(ppq.a, gpq, lds);
@@ -503,33 +486,20 @@ __global__ __launch_bounds__(kBlock) void k_mp_update(int n, int gpq, float *__r
     if (h.pq && c.iteration < h.cap) h.pq[c.iteration] = pq;
     if (h.alpha && c.iteration < h.cap) h.alpha[c.iteration] = alpha;
   }
-  Quads Q(n);
   double s_rr = 0.0;
-  for (; Q.q + (kQuadUnroll - 1) * Q.T < Q.full; Q.q += kQuadUnroll * Q.T) {
-    float4 rv[kQuadUnroll], qv[kQuadUnroll];
-#pragma unroll
-    for (int u = 0; u < kQuadUnroll; u++) {
-      const int64_t j = Q.q + u * Q.T;
-      rv[u] = v4(r)[j];
-      qv[u] = v4(q)[j];
-    }
-#pragma unroll
-    for (int u = 0; u < kQuadUnroll; u++) {
-      const int64_t j = Q.q + u * Q.T;
-      mp_update_elem(rv[u].x, qv[u].x, na, s_rr);
-      mp_update_elem(rv[u].y, qv[u].y, na, s_rr);
-      mp_update_elem(rv[u].z, qv[u].z, na, s_rr);
-      mp_update_elem(rv[u].w, qv[u].w, na, s_rr);
-      v4(r)[j] = rv[u];
-    }
-  }
-  for (; Q.q < Q.nquad; Q.q += Q.T) {
-    for (int64_t e = 4 * Q.q; e < 4 * Q.q + 4 && e < n; e++) {
+  quads.run([&](int64_t j, Quads2 &v) {
+    mp_update_elem(v.a.x, v.b.x, na, s_rr);
+    mp_update_elem(v.a.y, v.b.y, na, s_rr);
+    mp_update_elem(v.a.z, v.b.z, na, s_rr);
+    mp_update_elem(v.a.w, v.b.w, na, s_rr);
+    v4(r)[j] = v.a;
+  });
+  if (owns_rest(Q, Q.nquad))
+    for (int64_t e = 4 * Q.full; e < n; e++) {
       float re = r[e];
       mp_update_elem(re, q[e], na, s_rr);
       r[e] = re;
     }
-  }
   const double b0 = block_fold(s_rr, lds);
   if (threadIdx.x == 0) prr.a[blockIdx.x] = b0;
 }
@@ -537,41 +507,42 @@ __global__ __launch_bounds__(kBlock) void k_mp_update(int n, int gpq, float *__r
 // y32 += a p32 and p32 = u + b p32 over quads (the old p read once); y32,
 // read again only by a reliable update, is streamed non-temporally so that
 // p32 stays cached for the next SpMV.
-__device__ inline void mp_yp_update(int n, float *__restrict__ y, float *__restrict__ p,
-                                    const float *__restrict__ u, float a, float b) {
-  Quads Q(n);
-  for (; Q.q + (kQuadUnroll - 1) * Q.T < Q.full; Q.q += kQuadUnroll * Q.T) {
-    float4 yv[kQuadUnroll], pv[kQuadUnroll], uv[kQuadUnroll];
-#pragma unroll
-    for (int k = 0; k < kQuadUnroll; k++) {
-      const int64_t j = Q.q + k * Q.T;
-      yv[k] = v4_stream(y, j);
-      pv[k] = v4(p)[j];
-      uv[k] = v4(u)[j];
-    }
-#pragma unroll
-    for (int k = 0; k < kQuadUnroll; k++) {
-      const int64_t j = Q.q + k * Q.T;
+struct YpUpdate {
+  int n;
+  float *y, *p;
+  const float *u;
+  Quads Q;
+  __device__ YpUpdate(int m, float *yy, float *pp, const float *uu) : n(m), y(yy), p(pp), u(uu), Q(m) {}
+  // the first loads
+  __device__ __forceinline__ auto begin() const {
+    float *yy = y, *pp = p;
+    const float *uu = u;
+    return trips<kQuadUnroll>(
+        Q, [=](int64_t j) { return Quads3{v4_stream(yy, j), v4(pp)[j], v4(uu)[j]}; });
+  }
+  template <typename T>
+  __device__ __forceinline__ void run(T &quads, float a, float b) const {
+    quads.run([&](int64_t j, Quads3 &v) {
       float4 yo, po;
-      yo.x = yv[k].x + a * pv[k].x;
-      yo.y = yv[k].y + a * pv[k].y;
-      yo.z = yv[k].z + a * pv[k].z;
-      yo.w = yv[k].w + a * pv[k].w;
-      po.x = uv[k].x + b * pv[k].x;
-      po.y = uv[k].y + b * pv[k].y;
-      po.z = uv[k].z + b * pv[k].z;
-      po.w = uv[k].w + b * pv[k].w;
+      yo.x = v.a.x + a * v.b.x;
+      yo.y = v.a.y + a * v.b.y;
+      yo.z = v.a.z + a * v.b.z;
+      yo.w = v.a.w + a * v.b.w;
+      po.x = v.c.x + b * v.b.x;
+      po.y = v.c.y + b * v.b.y;
+      po.z = v.c.z + b * v.b.z;
+      po.w = v.c.w + b * v.b.w;
       v4_store_stream(y, j, yo);
       v4(p)[j] = po;
-    }
+    });
+    if (owns_rest(Q, Q.nquad))
+      for (int64_t e = 4 * Q.full; e < n; e++) {
+        const float pe = p[e];
+        y[e] = y[e] + a * pe;
+        p[e] = u[e] + b * pe;
+      }
   }
-  for (; Q.q < Q.nquad; Q.q += Q.T)
-    for (int64_t e = 4 * Q.q; e < 4 * Q.q + 4 && e < n; e++) {
-      const float pe = p[e];
-      y[e] = y[e] + a * pe;
-      p[e] = u[e] + b * pe;
-    }
-}
+};
 
 // Writes `next`: iteration count, rho = rz, r2 = rr, the inner residual and
 // the reliable-update trigger; the history entries.
@@ -592,18 +563,20 @@ __device__ inline void mp_advance(MixedState *st, const MixedScalars &c, double 
 
 // y32 += alpha p32 (alpha from the r update); beta = <r,r>_new / <r,r>;
 // p32 = r32 + beta p32 (always: a reliable update keeps p).  Writes `next`.
-__global__ __launch_bounds__(kBlock) void k_mp_xpay(int n, float *__restrict__ y,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_mp_xpay(int n, float *__restrict__ y,
                                                     float *__restrict__ p,
                                                     const float *__restrict__ r, Partials prr,
                                                     MixedState *st, History h) {
   __shared__ double lds[4];
+  const YpUpdate yp(n, y, p, r);
+  auto quads = yp.begin();
   const MixedScalars c = st->cur;
   if (c.done) return;
   const double rr = fold_partials(prr.a, gridDim.x, lds);  // the update ran on this grid
   const double beta = rr / c.rho;
   const float a = st->alpha32;
   if (blockIdx.x == 0 && threadIdx.x == 0) mp_advance(st, c, rr, rr, beta, h);
-  mp_yp_update(n, y, p, r, a, (float)beta);
+  yp.run(quads, a, (float)beta);
 }
 
 // ---------------------------------------------------------------------------
@@ -819,20 +792,23 @@ __global__ __launch_bounds__(kBlock) CGHIP_SGPR_CAP void k_mp_matvec_dot_quad(
 // y32 += alpha p32 (alpha from the r update); beta = <r,z>_new / <r,z>;
 // p32 = z + beta p32; stop test / reliable-update trigger on the inner
 // residual.  Writes `next`.
-__global__ __launch_bounds__(kBlock) void k_mp_xpay_poly(int n, float *__restrict__ y,
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) void k_mp_xpay_poly(int n, float *__restrict__ y,
                                                          float *__restrict__ p,
                                                          const float *__restrict__ z, Partials prr,
                                                          Partials prz, int gz, MixedState *st,
                                                          History h) {
   __shared__ double lds[4];
+  const YpUpdate yp(n, y, p, z);
+  auto quads = yp.begin();
   const MixedScalars c = st->cur;
   if (c.done) return;
   double rr, rz;
-  fold_partials2(prr.a, gridDim.x, prz.a, gz, lds, rr, rz);
+  // four at a time: the vectors' first loads hold the other registers
+  fold_partials2<4>(prr.a, gridDim.x, prz.a, gz, lds, rr, rz);
   const double beta = rz / c.rho;
   const float a = st->alpha32;
   if (blockIdx.x == 0 && threadIdx.x == 0) mp_advance(st, c, rr, rz, beta, h);
-  mp_yp_update(n, y, p, z, a, (float)beta);
+  yp.run(quads, a, (float)beta);
 }
 
 int row_grid(int n) {
