@@ -316,7 +316,8 @@ __global__ __launch_bounds__(kBlock) void k_fold_out(Partials pa, int G, int two
 }
 
 // k_dot_partials and k_fold_out in one block of 1,024 threads, for vectors of
-// at most kDotSmall pairs per thread: the loop of hooks waits for every dot,
+// 1 element to kDotSmall pairs per thread (its loads are clamped to the last
+// element, so an empty vector, whose pointers may be null, takes the two): the loop of hooks waits for every dot,
 // and a launch costs more than the rest of it (4,096 elements 13.7 us a call
 // against 16.1 with two kernels, 8,192 14.7, 16,384 17.0 against 16.1).  Wave
 // sums, partials and their fold are those of the two kernels, one pair per
@@ -793,7 +794,7 @@ hipError_t fill(int n, double v, double *y, hipStream_t s) {
 hipError_t dot_tree(int n, const double *a, const double *b, Partials pa, double *out,
                     hipStream_t s) {
   const int G = vec_grid(n);
-  if (G <= 4 * kDotSmall) {
+  if (n > 0 && G <= 4 * kDotSmall) {
     hipLaunchKernelGGL(k_dot_small, dim3(1), dim3(1024), 0, s, n, a, b, G, out);
     return hipGetLastError();
   }

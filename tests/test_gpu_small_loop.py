@@ -5,6 +5,8 @@ an odd or even iteration, the tolerance or the iteration limit -- and with odd
 batches.  Then <p, q> of the oracle around the partial counts at which the r
 update's own fold of them changes (one group, 2,048 partials).
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,27 @@ def test_dot_hook(ctx, n):
     ctx.upload("P", a)
     ctx.upload("Q", b)
     assert_bitwise([ctx.dot("P", "Q")], [oracle.lib().orc_dot_tree(n, a, b)], "<p, q>")
+
+
+@pytest.mark.parametrize("n", [0, 1, 5, 8192, 30001])
+def test_dot_without_allocation(ctx, n):
+    """Empty vectors (null pointers allowed) and vectors that start 8 bytes
+    past an aligned address."""
+    from cgxx_amd import cghip
+
+    L = cghip.load()
+    size = 30010
+    rng = np.random.default_rng(n + 1)
+    a, b = rng.standard_normal(size), rng.standard_normal(size)
+    ctx.set_size(size)
+    ctx.upload("P", a)
+    ctx.upload("R", b)
+    pa, pb, pz = ctx.pointer("P") + 8, ctx.pointer("R") + 8, ctx.pointer("Z")
+    if n == 0:
+        pa = pb = None
+    ctx.fill("Z", 7.0)
+    assert L.cghip_dot_noalloc(pa, pb, n, pz, None) == 0, L.cghip_last_error(None)
+    # the HIP runtime that the library itself is linked against (same soname)
+    assert C.CDLL("libamdhip64.so.7").hipDeviceSynchronize() == 0
+    want = oracle.lib().orc_dot_tree(n, a[1:n + 1].copy(), b[1:n + 1].copy()) if n else 0.0
+    assert_bitwise([ctx.download("Z")[0]], [want], "<a, b>")
