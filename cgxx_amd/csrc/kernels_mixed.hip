@@ -712,80 +712,73 @@ __global__ __launch_bounds__(kBlock) void k_poly_quad(Dia A, const float *__rest
                                        [](int, float, float) {});
 }
 
-// Rows of a dot, four per thread.  The block walks its chunks as
-// chunk_walk<true> says, four at a time: wave w takes rows 64 w .. 64 w + 63
-// of each of the four, 16 lanes a chunk; body(first row of the 16 lanes' 64,
-// lane among the 16, at) puts the contributions of its rows to at[0 .. 3].
-// Lane l of the wave then adds those of the
-// chunks' rows 64 w + l in walk order, so the partials are those of one row
-// per thread, and no barrier is needed (with a chunk per wave and a barrier
-// per four of them the CG product took 38.8 us at 187 x 201 x 190 against
-// 36.3, and as much at 256^3).
+// Rows of a dot, four per thread, and its partial (in lane 0).  A block of
+// one wave walks the chunks that chunk_walk<true> gives a block of 256: lane l
+// keeps the sums of threads 4 l .. 4 l + 3, which body(first row, lane, c)
+// extends by the rows' contributions c[0 .. 3], and the folds at the end are
+// those of the 256 threads.  The loop thus needs neither barriers nor LDS and
+// loads whole chunks.  With four chunks of a block at once, 64 rows of each to
+// a wave, and their contributions handed over through LDS: mixed Jacobi
+// iteration at 256^3 170.9 us instead of 168.4, and at 187 x 201 x 190 no
+// better than a row per thread.
 template <typename Body>
-__device__ inline double quad_dot_rows(int n, double (*place)[4][64], Body body) {
+__device__ inline double quad_dot_rows(int n, double *lds, Body body) {
   int rb0, stride, rend;
   chunk_walk<true>(ell_chunks(n), rb0, stride, rend);
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, seg = lane >> 4, g = lane & 15;
-  double(*mine)[64] = place[wave];
-  double tpart = 0.0;
-  for (int rb = rb0; rb < rend; rb += 4 * stride) {
-    const int c = rb + seg * stride;
-    if (c < rend) body(c * kBlock + 64 * wave, g, &mine[seg][4 * g]);
-    // the wave's own slots: written and read in order
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int lane = threadIdx.x;
+  double sum[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int rb = rb0; rb < rend; rb += stride) {
+    const int r0 = rb * kBlock + 4 * lane;
+    double c[4];
+    body(r0, lane, c);
 #pragma unroll
-    for (int w = 0; w < 4; w++) {
-      const double v = mine[w][lane];
-      const int cw = rb + w * stride;
-      tpart = cw < rend && cw * kBlock + (int)threadIdx.x < n ? tpart + v : tpart;
-    }
-    __builtin_amdgcn_wave_barrier();
+    for (int e = 0; e < 4; e++) sum[e] = r0 + e < n ? sum[e] + c[e] : sum[e];
   }
-  return tpart;
+#pragma unroll
+  for (int e = 0; e < 4; e++) lds[4 * lane + e] = sum[e];
+  __syncthreads();
+  double w[4];
+#pragma unroll
+  for (int k = 0; k < 4; k++) w[k] = wave_fold(lds[64 * k + lane]);
+  return ((w[0] + w[1]) + w[2]) + w[3];
 }
 
 // The last step (j = 0): z and the partials of <r, z>.
-template <int MODE, bool UNIT>
-__global__ __launch_bounds__(kBlock) CGHIP_SGPR_CAP void k_poly_quad_dot(
+template <int MODE, bool NT, bool UNIT>
+__global__ __launch_bounds__(64) CGHIP_SGPR_CAP void k_poly_quad_dot(
     Dia A, const float *__restrict__ b1, const float *__restrict__ b2, const float *__restrict__ r,
     const PolyParams *poly, float *__restrict__ b0, float *__restrict__ pcopy, Partials prz,
     const MixedState *st) {
-  __shared__ double place[4][4][64];
-  __shared__ double lds[4];
+  __shared__ double lds[kBlock];
   if (st && st->cur.done) return;
-  const double tpart = quad_dot_rows(A.n, place, [&](int s0, int g, double *at) {
-    poly_quad<true, MODE, true, UNIT, 16>(
-        A, b1, b2, r, poly, 0, s0 + 4 * g, g, b0, pcopy,
-        [at](int e, float ri, float z) { at[e] = (double)ri * (double)z; });
+  const double bp = quad_dot_rows(A.n, lds, [&](int r0, int lane, double *c) {
+    poly_quad<true, MODE, NT, UNIT, 64>(
+        A, b1, b2, r, poly, 0, r0, lane, b0, pcopy,
+        [c](int e, float ri, float z) { c[e] = (double)ri * (double)z; });
   });
-  const double bp = block_fold(tpart, lds);
   if (threadIdx.x == 0) prz.a[blockIdx.x] = bp;
 }
 
 // k_mp_matvec_dot on the upper diagonals of a symmetric FP32 DIA operator,
-// four rows per thread: 20 bytes a row instead of 32.  256^3 100 -> 83 us
-// (4.1 TB/s; the loop's vectors and values outgrow the last-level cache).
+// four rows per thread: 20 bytes a row instead of 32.  256^3 100 -> 78 us in
+// the loop, whose vectors and values outgrow the last-level cache (4.6 TB/s,
+// what a large copy reaches).
 template <bool UNIT>
-__global__ __launch_bounds__(kBlock) CGHIP_SGPR_CAP void k_mp_matvec_dot_quad(
+__global__ __launch_bounds__(64) CGHIP_SGPR_CAP void k_mp_matvec_dot_quad(
     Dia A, const float *__restrict__ p, float *__restrict__ q, Partials pq, MixedState *st) {
-  __shared__ double place[4][4][64];
-  __shared__ double lds[4];
+  __shared__ double lds[kBlock];
   if (!mp_begin(st)) return;
-  const double tpart = quad_dot_rows(A.n, place, [&](int s0, int g, double *at) {
-    const int r0 = s0 + 4 * g;
+  const double bp = quad_dot_rows(A.n, lds, [&](int r0, int lane, double *c) {
     DiaQuad<uint32_t> l;
-    dia_quad_load<uint32_t, UNIT, 16>(A, p, r0, g, l);
+    dia_quad_load<uint32_t, UNIT, 64>(A, p, r0, lane, l);
     f4 o;
 #pragma unroll
     for (int e = 0; e < 4; e++) {
       o[e] = l.own[e] + dia_quad_sum(l, e);
-      at[e] = (double)l.own[e] * (double)o[e];
+      c[e] = (double)l.own[e] * (double)o[e];
     }
     reinterpret_cast<f4 *>(q)[r0 >> 2] = o;
   });
-  const double bp = block_fold(tpart, lds);
   if (threadIdx.x == 0) pq.a[blockIdx.x] = bp;
 }
 
@@ -956,20 +949,26 @@ static void poly_apply_half(const Op32 &A, const float *r32, const PolyParams *p
     poly_apply_t<kOpDia, true, false, 2>(A, r32, poly, degree, w, pcopy, prz, st, s);
 }
 
-// Its last step: four rows per thread where the step streams (NT), else one
-// (first and last step 128^3 7.6 us with one, 9.5 with four, 187 x 201 x 190
-// 24.0 and 25.2, 224^3 36.9 and 38.2; 240^3 52.4 and 45.4, 256^3 58.7 and 48.8).
+// Whether a dot takes four rows per thread: where a partial has more than
+// four chunks.  One wave then walks them; with fewer chunks a block of four
+// waves, a row per thread, is the faster (first and last Clenshaw step and
+// mixed Jacobi iteration, a row and four: 110^3 6.1 and 6.4, 26.2 and 26.7 us,
+// 128^3 7.5 and 7.7, 32.2 and 32.5; 187 x 201 x 190 24.0 and 21.1, 79.4 and
+// 76.5, 224^3 36.8 and 31.9, 118.7 and 116.1).
+static bool quad_dots(const Dia &d) { return ell_chunks(d.n) > 4 * dia_grid(d.n); }
+
+// The last step on the symmetric FP16 streams.
 template <int MODE, bool NT, bool UNIT>
 static void poly_last_sym(const Op32 &A, const float *b1, const float *b2, const float *r32,
                           const PolyParams *poly, float *b0, float *pcopy, Partials prz,
                           const MixedState *st, hipStream_t s) {
-  const dim3 grid(op32_grid(A)), block(kBlock);
-  if constexpr (NT)
-    hipLaunchKernelGGL((k_poly_quad_dot<MODE, UNIT>), grid, block, 0, s, A.dia, b1, b2, r32, poly, b0,
-                       pcopy, prz, st);
+  const dim3 grid(op32_grid(A));
+  if (quad_dots(A.dia))
+    hipLaunchKernelGGL((k_poly_quad_dot<MODE, NT, UNIT>), grid, dim3(64), 0, s, A.dia, b1, b2, r32,
+                       poly, b0, pcopy, prz, st);
   else
-    hipLaunchKernelGGL((k_poly_step<true, kOpDia, MODE, true, false, 2, true>), grid, block, 0, s, A,
-                       b1, b2, r32, poly, 0, b0, pcopy, prz, st);
+    hipLaunchKernelGGL((k_poly_step<true, kOpDia, MODE, true, false, 2, true>), grid, dim3(kBlock), 0,
+                       s, A, b1, b2, r32, poly, 0, b0, pcopy, prz, st);
 }
 
 // The steps on the symmetric FP16 streams.
@@ -1054,14 +1053,12 @@ hipError_t mp_matvec_dot(const Op32 &A, const float *p, float *q, Partials pq, M
   switch (A.kind) {
     case kOpDia:
       if (A.dia.unit != 1) return hipErrorInvalidValue;
-      // as the Clenshaw steps' last: 128^3 product 13.7 us with four rows per
-      // thread, 12.8 with one, 224^3 56.2 both, 240^3 70.7 and 73.7, 256^3
-      // 82.6 and 90.1; from all six streams 18.9, 68.9, 88.4 and 100.4
-      if (A.dia.sym32 && A.dia.pad && poly_stream_sym(A.dia.n)) {
+      if (A.dia.sym32 && A.dia.pad && quad_dots(A.dia)) {
+        const dim3 wave(64);
         if (quad_unit(A.dia))
-          hipLaunchKernelGGL(k_mp_matvec_dot_quad<true>, grid, block, 0, s, A.dia, p, q, pq, st);
+          hipLaunchKernelGGL(k_mp_matvec_dot_quad<true>, grid, wave, 0, s, A.dia, p, q, pq, st);
         else
-          hipLaunchKernelGGL(k_mp_matvec_dot_quad<false>, grid, block, 0, s, A.dia, p, q, pq, st);
+          hipLaunchKernelGGL(k_mp_matvec_dot_quad<false>, grid, wave, 0, s, A.dia, p, q, pq, st);
       } else if (A.dia.sym32)
         hipLaunchKernelGGL((k_mp_matvec_dot<kOpDia, true>), grid, block, 0, s, A, p, q, pq, st);
       else
