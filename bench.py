@@ -84,6 +84,12 @@ def kernel_short_name(name: str) -> str:
     return name
 
 
+def sym64_bytes(n: int, ndiag: int) -> int:
+    """FP64 product on the symmetric diagonals: the diagonal and half of the
+    ndiag others, x and y."""
+    return 8 * (1 + ndiag // 2) * n + 16 * n
+
+
 def algorithmic_bytes(short: str, meta: dict):
     """Bytes a launch must move at least (each array once, x once per SpMV)."""
     n, nnz, D = meta["n"], meta["nnz"], meta["ndiag"]
@@ -94,8 +100,9 @@ def algorithmic_bytes(short: str, meta: dict):
     rec = D * n if len(args) >= 7 and args[6] == "true" else 4 * ((D + 1) // 2) * n
     table = [("k_pcg_matvec_dot_crs", crs_bytes(n, nnz, 8, 8)), ("k_matvec_crs<double", crs_bytes(n, nnz, 8, 8)),
              ("k_pcg_matvec_dot_ell", ell_bytes(n, nnz, 8, 8)), ("k_matvec_ell<double", ell_bytes(n, nnz, 8, 8)),
-             ("k_pcg_update<true>", 32 * n), ("k_pcg_update<false>", 24 * n), ("k_pcg_xpay<true>", 48 * n),
-             ("k_pcg_xpay<false>", 40 * n), ("k_mp_matvec_dot<2, true", 2 * D * n + 8 * n),
+             ("k_pcg_matvec_dot_sym64", sym64_bytes(n, D)), ("k_matvec_sym64", sym64_bytes(n, D)),
+             ("k_pcg_update<true", 32 * n), ("k_pcg_update<false", 24 * n), ("k_pcg_xpay<true", 48 * n),
+             ("k_pcg_xpay<false", 40 * n), ("k_mp_matvec_dot<2, true", 2 * D * n + 8 * n),
              ("k_mp_matvec_dot_quad", 2 * D * n + 8 * n), ("k_mp_matvec_dot<2", 4 * D * n + 8 * n),
              ("k_poly_quad<1,", D * n + 8 * n), ("k_poly_quad<2,", D * n + 12 * n),
              ("k_poly_quad<0,", D * n + 16 * n), ("k_poly_quad_dot<0,", D * n + 16 * n),
@@ -237,10 +244,11 @@ def application_traffic(kind: int, degree: int):
     """PMC bytes per Clenshaw step averaged over one application: the first
     step (template arguments <false, kind, 1, ...>), the second (2), the
     plain ones (0) and the last (final, 0)."""
-    first = traffic_from_profiles(f"k_poly_step<false, {kind}, 1,")
-    second = traffic_from_profiles(f"k_poly_step<false, {kind}, 2,")
-    plain = traffic_from_profiles(f"k_poly_step<false, {kind}, 0,")
-    last = traffic_from_profiles(f"k_poly_step<true, {kind}, 0,")
+    # four rows per thread where the symmetric storage runs them, else one
+    first, second, plain = (traffic_from_profiles(f"k_poly_quad<{mode},") or
+                            traffic_from_profiles(f"k_poly_step<false, {kind}, {mode},")
+                            for mode in (1, 2, 0))
+    last = traffic_from_profiles("k_poly_quad_dot<0,") or traffic_from_profiles(f"k_poly_step<true, {kind}, 0,")
     if degree < 3 or None in (first, second, plain, last):
         return None
     return (first + second + (degree - 3) * plain + last) / degree
@@ -479,7 +487,10 @@ def main() -> int:
         xs[fmt] = ctx.download("X")
         prof = run64(profile=1)
         spmv_ms = per(prof, "matvec")
-        by = crs_bytes(n, nnz, 8, 8) if fmt == "CRS" else ell_bytes(n, nnz, 8, 8)
+        # the stencil is symmetric bit for bit: its products read the symmetric
+        # diagonals in both formats
+        by = sym64_bytes(n, ndiag) if 0 < ndiag <= 6 else \
+            crs_bytes(n, nnz, 8, 8) if fmt == "CRS" else ell_bytes(n, nnz, 8, 8)
         plain_ms = ctx.time_matvec("P", "Q", reps=20)
         fp64[fmt] = {
             "seconds": sec, "iterations": info["iterations"], "true_relative_residual": nr / nb,
@@ -638,7 +649,7 @@ def main() -> int:
             "unit": "GB/s",
             "frac": step_gbps / HBM_PEAK_GBS,
             "traffic": application_traffic(kind, deg),
-            "kernel": f"k_poly_step<*, {kind}, *>: the Clenshaw steps of one degree-{deg} application, "
+            "kernel": f"k_poly_quad / k_poly_step<*, {kind}, *>: the Clenshaw steps of one degree-{deg} application, "
                       f"per step (scaled operator in {layout}"
                       + (", FP16 values)" if layout == "DIA" else ", FP32 values)"),
             "polynomial": prof_src,
