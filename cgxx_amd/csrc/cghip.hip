@@ -80,7 +80,7 @@ struct cghip_ctx {
 
   // mixed precision: the FP32 copy of the CRS values; the scaled operator
   // D^-1/2 A D^-1/2 with implicit unit diagonal (off-diagonal CRS + its row
-  // blocks, s = 1/sqrt(diag) in FP64); FP32 work vectors y32, r32, p32, q32;
+  // blocks only where no layout below holds it, s = 1/sqrt(diag) in FP64); FP32 work vectors y32, r32, p32, q32;
   // the inner loop's state and graph
   bool has_fp32 = false;
   float *value32 = nullptr;

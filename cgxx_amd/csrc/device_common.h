@@ -543,9 +543,8 @@ __device__ inline double dia_row_pre_epi(const Dia &A, const float *__restrict__
 // Four consecutive rows per thread of a DIA operator whose kSymPairs mirrored
 // pairs of diagonals equal their transposes bit for bit: V = uint16_t reads
 // the streams Dia::up16, V = uint32_t the upper diagonals of Dia::val; row
-// i's lower entries are those of rows i - o.  G neighbouring lanes (64 or 16)
-// hold 4 G consecutive rows.  A row's products and their order are those of
-// dia_row_finish.
+// i's lower entries are those of rows i - o.  A wave holds 256 consecutive
+// rows.  A row's products and their order are those of dia_row_finish.
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint16_t h4 __attribute__((ext_vector_type(4)));
@@ -568,17 +567,13 @@ struct QuadOf<uint32_t> {
   typedef u4_any any;
 };
 
-// The value of the lane before (after) of a group of G lanes, `edge` in its
-// first (last) lane.  Every lane of the group is active.
-template <int G>
+// The value of the lane before (after), `edge` in the wave's first (last)
+// lane.  Every lane is active.
 __device__ inline uint32_t lane_before(uint32_t v, uint32_t edge) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, G == 64 ? 0x138 : 0x111, 0xf, 0xf,
-                                               false);
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, 0x138, 0xf, 0xf, false);
 }
-template <int G>
 __device__ inline uint32_t lane_after(uint32_t v, uint32_t edge) {
-  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, G == 64 ? 0x130 : 0x101, 0xf, 0xf,
-                                               false);
+  return (uint32_t)__builtin_amdgcn_update_dpp((int)edge, (int)v, 0x130, 0xf, 0xf, false);
 }
 
 template <typename V>
@@ -587,15 +582,15 @@ struct DiaQuad {
   f4 own, xl[kSymPairs], xh[kSymPairs];
 };
 
-// All loads of rows r0 .. r0 + 3 of the lane, the g-th of its group.  Dia::pad
+// All loads of rows r0 .. r0 + 3 of the lane.  Dia::pad
 // keeps them inside the allocations for every row of a tile, those before row
 // 0 and past the last one too; what lies there is dropped: an upper entry
 // past the matrix is absent, and a lower one before it is marked absent here.
 // UNIT (the nearest pair is +-1): x at r +- 1 and its lower value come from
 // the thread's own quad and its neighbour lanes', and one load for the two
 // ends of the group, instead of three more quads.
-template <typename V, bool UNIT, int G>
-__device__ inline void dia_quad_load(const Dia &A, const float *__restrict__ x, int r0, int g,
+template <typename V, bool UNIT>
+__device__ inline void dia_quad_load(const Dia &A, const float *__restrict__ x, int r0, int lane,
                                      DiaQuad<V> &l) {
   typedef typename QuadOf<V>::any Any;
   constexpr uint32_t B = sizeof(V);
@@ -622,14 +617,14 @@ __device__ inline void dia_quad_load(const Dia &A, const float *__restrict__ x, 
     l.xh[k] = xs(r0 + o);
   }
   if (UNIT) {
-    const int before = r0 - 4 * g - 1;
-    const uint32_t xe = *reinterpret_cast<const uint32_t *>(xp + at(g == G - 1 ? r0 + 4 : before, 4u));
+    const int before = r0 - 4 * lane - 1;
+    const uint32_t xe = *reinterpret_cast<const uint32_t *>(xp + at(lane == 63 ? r0 + 4 : before, 4u));
     const uint32_t le = *reinterpret_cast<const V *>(up + at(before, B));
-    const uint32_t xa = lane_before<G>(__float_as_uint(l.own.w), xe);
-    const uint32_t xz = lane_after<G>(__float_as_uint(l.own.x), xe);
+    const uint32_t xa = lane_before(__float_as_uint(l.own.w), xe);
+    const uint32_t xz = lane_after(__float_as_uint(l.own.x), xe);
     l.xl[0] = f4{__uint_as_float(xa), l.own.x, l.own.y, l.own.z};
     l.xh[0] = f4{l.own.y, l.own.z, l.own.w, __uint_as_float(xz)};
-    l.lo[0].x = (V)lane_before<G>((uint32_t)l.up[0].w, le);
+    l.lo[0].x = (V)lane_before((uint32_t)l.up[0].w, le);
     l.lo[0].y = l.up[0].x;
     l.lo[0].z = l.up[0].y;
     l.lo[0].w = l.up[0].z;

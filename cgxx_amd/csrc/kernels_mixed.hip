@@ -655,13 +655,13 @@ __device__ inline float clenshaw(float t0, float bi, float ri, float bb, float c
   return FINAL ? (cj * ri + sv) - bb : (cj * ri + 2.0f * sv) - bb;
 }
 
-// The Clenshaw rows r0 .. r0 + 3 of a lane, the g-th of a group of G, on the
-// symmetric FP16 streams: out(e, r, B_j) for each of them.  Rows past the
-// last are computed too, into the padding (Dia::pad).
-template <bool FINAL, int MODE, bool NT, bool UNIT, int G, typename Out>
+// The Clenshaw rows r0 .. r0 + 3 of a lane on the symmetric FP16 streams:
+// out(e, r, B_j) for each of them.  Rows past the last are computed too, into
+// the padding (Dia::pad).
+template <bool FINAL, int MODE, bool NT, bool UNIT, typename Out>
 __device__ inline void poly_quad(const Dia &A, const float *__restrict__ b1,
                                  const float *__restrict__ b2, const float *__restrict__ r,
-                                 const PolyParams *poly, int j, int r0, int g,
+                                 const PolyParams *poly, int j, int r0, int lane,
                                  float *__restrict__ b0, float *__restrict__ pcopy, Out out) {
   const float cj = poly->c[j], tb = poly->two_over_b, ck = poly->c[poly->degree];
   const int q = r0 >> 2;
@@ -673,7 +673,7 @@ __device__ inline void poly_quad(const Dia &A, const float *__restrict__ b1,
   f4 rv, bv;
   if (MODE != kStepFirst) rv = quad(r);
   if (MODE == kStepPlain) bv = quad(b2);
-  dia_quad_load<uint16_t, UNIT, G>(A, MODE == kStepFirst ? r : b1, r0, g, l);
+  dia_quad_load<uint16_t, UNIT>(A, MODE == kStepFirst ? r : b1, r0, lane, l);
   if (MODE == kStepFirst) rv = l.own;
   f4 o;
 #pragma unroll
@@ -708,7 +708,7 @@ __global__ __launch_bounds__(kBlock) void k_poly_quad(Dia A, const float *__rest
   const int w0 = __builtin_amdgcn_readfirstlane(tile * 1024 + (int)(threadIdx.x >> 6) * 256);
   if (w0 >= A.n) return;
   const int lane = threadIdx.x & 63;
-  poly_quad<false, MODE, NT, UNIT, 64>(A, b1, b2, r, poly, j, w0 + 4 * lane, lane, b0, nullptr,
+  poly_quad<false, MODE, NT, UNIT>(A, b1, b2, r, poly, j, w0 + 4 * lane, lane, b0, nullptr,
                                        [](int, float, float) {});
 }
 
@@ -752,7 +752,7 @@ __global__ __launch_bounds__(64) CGHIP_SGPR_CAP void k_poly_quad_dot(
   __shared__ double lds[kBlock];
   if (st && st->cur.done) return;
   const double bp = quad_dot_rows(A.n, lds, [&](int r0, int lane, double *c) {
-    poly_quad<true, MODE, NT, UNIT, 64>(
+    poly_quad<true, MODE, NT, UNIT>(
         A, b1, b2, r, poly, 0, r0, lane, b0, pcopy,
         [c](int e, float ri, float z) { c[e] = (double)ri * (double)z; });
   });
@@ -770,7 +770,7 @@ __global__ __launch_bounds__(64) CGHIP_SGPR_CAP void k_mp_matvec_dot_quad(
   if (!mp_begin(st)) return;
   const double bp = quad_dot_rows(A.n, lds, [&](int r0, int lane, double *c) {
     DiaQuad<uint32_t> l;
-    dia_quad_load<uint32_t, UNIT, 64>(A, p, r0, lane, l);
+    dia_quad_load<uint32_t, UNIT>(A, p, r0, lane, l);
     f4 o;
 #pragma unroll
     for (int e = 0; e < 4; e++) {

@@ -129,7 +129,9 @@ int cghip_dot_noalloc(const double *a, const double *b, int n, double *out,
 /* --- fused solver ----------------------------------------------------------
  * The whole loop of CG::solve (CG.cpp:284-385) on the device: three kernels
  * per iteration (SpMV + <p,q>; r update + <r,r> + <r,z>; x += a p and
- * p = C r + b p).
+ * p = C r + b p), or two with the same results where the system is small and
+ * its matrix a symmetric stencil (the last of an iteration and the first of
+ * the next in one; not with CGHIP_PROFILE_KERNELS).
  * Each kernel writes per-block partial sums; the next kernel folds them (in
  * a fixed order) and computes alpha, beta and the stop test itself, so no
  * host round trip is needed per iteration.  Iterations are replayed from a
