@@ -223,8 +223,7 @@ void free_fp32(cghip_ctx *c) {
 }
 
 void free_sym(Sym64 &s) {
-  if (s.diag) (void)hipFree((void *)s.diag);
-  if (s.up) (void)hipFree((void *)s.up);
+  if (s.diag) (void)hipFree((void *)s.diag);  // up lies in the same allocation
   s = Sym64{};
 }
 
@@ -365,7 +364,9 @@ int row_blocks(int n, const int *ptr, int longest, std::vector<int> &rb) {
 // one before; without the memory for both at once it stays null and the
 // caller looks the indices over itself (*in_range false).  The check on the
 // device reads the copy in 20 us where a loop on the host took 5 ms (14.6
-// million entries).
+// million entries); the caller looks over short arrays itself too, up to
+// kHostCheck entries, which takes as long as the flag's way back.
+constexpr int64_t kHostCheck = 1 << 16;
 template <typename Check>
 int copy_columns(cghip_ctx *c, const int *index, int64_t count, int **copy, bool *in_range,
                  Check check) {
@@ -373,6 +374,7 @@ int copy_columns(cghip_ctx *c, const int *index, int64_t count, int **copy, bool
   *in_range = true;
   if (count == 0) return CGHIP_OK;
   *in_range = false;
+  if (count <= kHostCheck) return CGHIP_OK;
   int *d = nullptr;
   if (hipMalloc((void **)&d, sizeof(int) * (size_t)count) != hipSuccess) {
     (void)hipGetLastError();
@@ -433,13 +435,13 @@ int build_sym(cghip_ctx *c, const M &A, const Offsets &o, Sym64 *out) {
   for (int k = 0; k < S.pairs; k++) S.off[k] = o.off[S.pairs + k];
   int *found = reinterpret_cast<int *>(c->partial);
   double *diag = nullptr, *up = nullptr;
+  const size_t rows = ((size_t)A.n + 63) / 64 * 64;
   const size_t streams = (size_t)S.pairs * ((size_t)A.n + kSym64Pad);
-  if (hipMalloc((void **)&diag, sizeof(double) * (size_t)A.n) != hipSuccess ||
-      hipMalloc((void **)&up, sizeof(double) * streams) != hipSuccess) {
+  if (hipMalloc((void **)&diag, sizeof(double) * (rows + streams)) != hipSuccess) {
     (void)hipGetLastError();
-    if (diag) (void)hipFree(diag);
     return CGHIP_OK;
   }
+  up = diag + rows;
   S.diag = diag;
   S.up = up;
   int bad = 1;

@@ -1,4 +1,5 @@
-"""Uploads whose columns the device checks: a refused matrix names its first
+"""Uploads whose columns are checked, on the device above 65,536 entries (the
+largest n below), else on the host: a refused matrix names its first
 bad entry and leaves the one before, for both formats; and the scaled operator
 in CRS around the row length (8 off-diagonal entries) from which its row blocks
 are no longer whole chunks.
@@ -23,7 +24,7 @@ def ctx():
 
 
 @pytest.mark.parametrize("fmt", ["CRS", "ELL"])
-@pytest.mark.parametrize("n", [2, 257, 4096])
+@pytest.mark.parametrize("n", [2, 257, 4096, 40000])
 def test_refused_matrix_leaves_the_one_before(ctx, n, fmt):
     from cgxx_amd.cghip import CGHIPError
 
