@@ -9,6 +9,7 @@
 
 #include "../../include/cghip.h"
 #include "cghip_kernels.h"
+#include "crs_rows.h"
 #include "matrix_stats.h"
 
 #include <algorithm>
@@ -576,15 +577,9 @@ int cghip_upload_crs(cghip_ctx *c, int n, int nnz, const int32_t *ptr, const int
     return fail(c, CGHIP_ERR_ARG, "invalid CRS arguments (n=%d, nnz=%d)", n, nnz);
   if (ptr[0] != 0 || ptr[n] != nnz)
     return fail(c, CGHIP_ERR_ARG, "CRS ptr must start at 0 and end at nnz");
-  int shortest = INT32_MAX, longest = 0;
-  for (int i = 0; i < n; i++) {
-    const int len = (int)((uint32_t)ptr[i + 1] - (uint32_t)ptr[i]);  // wraps only past a decrease
-    shortest = std::min(shortest, len);
-    longest = std::max(longest, len);
-  }
-  if (shortest < 0)
-    for (int i = 0; i < n; i++)
-      if (ptr[i + 1] < ptr[i]) return fail(c, CGHIP_ERR_ARG, "CRS ptr decreases at row %d", i);
+  int longest = 0;
+  if (const int i = crs_rows(n, ptr, &longest); i >= 0)
+    return fail(c, CGHIP_ERR_ARG, "CRS ptr decreases at row %d", i);
   HIPCHK(c, hipSetDevice(c->device));
   int *new_index = nullptr;
   bool in_range = true;

@@ -104,3 +104,23 @@ def test_scaled_crs_rows(ctx, hub):
     assert info["iterations"] == oinfo["iterations"] == 6
     assert_bitwise(ctx.history("pq", 6), oh["pq"], "<p, q>")
     assert_bitwise(ctx.download("X"), ox, "x")
+
+
+@pytest.mark.parametrize("ptr, row", [([0, 2_000_000_000, -2_000_000_000, 0, 4], 1),
+                                      ([0, 1, 2_000_000_000, -2_000_000_000, 4], 2)])
+def test_decrease_that_wraps_is_refused(ctx, ptr, row):
+    """A row pointer that falls by more than 2^31: its 32-bit row lengths are
+    all positive.  The refusal comes from the host, before any launch."""
+    from cgxx_amd.cghip import CGHIPError
+
+    m = banded(4, (1,), 3)
+    ctx.set_size(4)
+    ctx.upload_crs(*m)
+    ctx.set_format("CRS")
+    ctx.upload("P", np.arange(1.0, 5.0))
+    ctx.matvec("P", "Q")
+    want = ctx.download("Q")
+    with pytest.raises(CGHIPError, match=f"decreases at row {row}$"):
+        ctx.upload_crs(np.array(ptr, np.int32), np.zeros(4, np.int32), np.ones(4))
+    ctx.matvec("P", "Q")
+    assert_bitwise(ctx.download("Q"), want, "product of the matrix before")
