@@ -140,3 +140,43 @@ def test_product_and_loop_bitwise(ctx, name, fmt):
     assert info["iterations"] == oit
     assert_bitwise(ctx.history("pq", oit), oh["pq"], "<p, q>")
     assert_bitwise(ctx.download("X"), ox, "x")
+
+
+@pytest.mark.parametrize("fmt", ["CRS", "ELL"])
+@pytest.mark.parametrize("at", [0, 256, 20000, 39999])
+def test_one_row_out_of_order(ctx, at, fmt):
+    """One block of 157 meets a row whose columns do not ascend: the row's
+    products are added as stored."""
+    n = 40000
+    ptr, index, value = (a.copy() for a in banded(n, (1, 200), 16, drop=0.0))
+    s = slice(ptr[at], ptr[at + 1])
+    index[s], value[s] = index[s][::-1].copy(), value[s][::-1].copy()
+    m = ptr, index, value
+    upload(ctx, m, fmt)
+    x = np.random.default_rng(at).standard_normal(n)
+    ctx.upload("P", x)
+    ctx.matvec("P", "Q")
+    assert_bitwise(ctx.download("Q"), reference_product(m, fmt, x), "product")
+
+
+@pytest.mark.parametrize("extra, layout", [(0, "DIA"), (1, "ELL")])
+def test_offsets_of_different_blocks(ctx, extra, layout):
+    """Offsets +-1 and +-2 in the rows of the first half, +-5 and +-9 in the
+    others: eight diagonals that no single block has; a ninth is too many."""
+    n = 40000
+    i = np.arange(n)
+    off = np.where((i < n // 2)[:, None], [[-2, -1, 0, 1, 2]], [[-9, -5, 0, 5, 9]])
+    col = i[:, None] + off
+    col[n - 1, 1] += extra  # offset -4
+    live = (col >= 0) & (col < n)
+    value = np.where(off == 0, 9.0, -np.random.default_rng(3).random((n, 5)))
+    ptr = np.zeros(n + 1, np.int32)
+    ptr[1:] = np.cumsum(live.sum(1))
+    m = ptr, col[live].astype(np.int32), value[live]
+    upload(ctx, m, "CRS")
+    ctx.prepare_fp32()
+    assert ctx.fp32_layout() == layout
+    x = np.random.default_rng(4).standard_normal(n)
+    ctx.upload("P", x)
+    ctx.matvec("P", "Q")
+    assert_bitwise(ctx.download("Q"), reference_product(m, "CRS", x), "product")
