@@ -933,8 +933,7 @@ static bool poly_rows4(const Op32 &A) {
   return (int64_t)ell_chunks(A.dia.n) >= 8 * (int64_t)op32_grid(A);
 }
 
-// The FP16 DIA steps with a row per thread: on the records, or on the
-// upper-diagonal streams of a system too small for quads (SYM).
+// The FP16 DIA steps on the records, a row per thread.
 static void poly_apply_half(const Op32 &A, const float *r32, const PolyParams *poly, int degree,
                             float *const w[3], float *pcopy, Partials prz, const MixedState *st,
                             hipStream_t s) {
@@ -1003,10 +1002,21 @@ static bool quad_unit(const Dia &d) { return d.off[kSymPairs] == 1; }
 static void poly_apply_sym(const Op32 &A, const float *r32, const PolyParams *poly, int degree,
                            float *const w[3], float *pcopy, Partials prz, const MixedState *st,
                            hipStream_t s) {
+  // No padding (quad_pad): at most 4,096 chunks, or a slab of any size, whose
+  // farthest pair lies beyond n / 8.  A row per thread, two a trip (four: the
+  // same times); non-temporal r and B_{j+2} from 12.9M rows on: step at 7 x
+  // 1344 x 1344 (12.6M) 48.8 us cached, 51.1 non-temporal, 7 x 1370 x 1380
+  // (13.2M) 64.9 and 62.1, 7 x 1600 x 1600 82.4 and 73.7, 3 x 2500 x 2500
+  // 106.7 and 93.3.
+  if (!A.dia.pad) {
+    if (22 * (int64_t)A.dia.n > 17 * (int64_t(1) << 24))
+      poly_apply_t<kOpDia, true, true, 2, true>(A, r32, poly, degree, w, pcopy, prz, st, s);
+    else
+      poly_apply_t<kOpDia, true, false, 2, true>(A, r32, poly, degree, w, pcopy, prz, st, s);
+    return;
+  }
   const bool nt = poly_stream_sym(A.dia.n);
-  if (!A.dia.pad)
-    poly_apply_t<kOpDia, true, false, 2, true>(A, r32, poly, degree, w, pcopy, prz, st, s);
-  else if (quad_unit(A.dia))
+  if (quad_unit(A.dia))
     nt ? poly_apply_quad<true, true>(A, r32, poly, degree, w, pcopy, prz, st, s)
        : poly_apply_quad<false, true>(A, r32, poly, degree, w, pcopy, prz, st, s);
   else

@@ -98,6 +98,22 @@ def test_quad_dots_bitwise(ctx, shape, degree):
     _compare(ctx, *_grid(*shape), iters=2, degree=degree)
 
 
+# slabs of fewer than 8 planes have no padding at any size and keep a row per
+# thread: cached, and above 12.96M rows non-temporal, without strips and with
+# them (a plane of 7,744 chunks)
+@pytest.mark.parametrize("degree", [1, 2, 4])
+@pytest.mark.parametrize("shape", [(7, 600, 600, 1), (7, 1371, 1367, 1), (7, 1408, 1408, 1)])
+def test_slabs_bitwise(ctx, shape, degree):
+    _compare(ctx, *_grid(*shape), iters=2, degree=degree)
+
+
+# planes of whole tiles: the steps' strip order, cached (a plane of 80 chunks)
+# and non-temporal (of 256)
+@pytest.mark.parametrize("shape", [(64, 128, 160, 1), (192, 256, 256, 1)])
+def test_strip_order_bitwise(ctx, shape):
+    _compare(ctx, *_grid(*shape), iters=2, degree=4)
+
+
 def test_fp32_values_not_symmetric(ctx):
     ptr, index, value = _grid(24, 23, 25)
     row = 24 * 23 * 25 // 2
