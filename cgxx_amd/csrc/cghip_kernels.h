@@ -151,9 +151,12 @@ constexpr int kSym64Pad = 1088;
 // matrix_bytes a row and five vectors, outgrow the 256 MB last-level cache.
 // Iteration on the symmetric diagonals of 128^3 (151 MB) 57 cached against
 // 66 us, 145 x 150 x 155 (243 MB) 82 against 95, 160^3 (295 MB) 116 against
-// 112, 256^3 481 against 429.
+// 112, 256^3 481 against 429.  And only above 2^21 rows: the vectors of a
+// shorter system, 80 MB at most, stay cached beside long rows (27-point ELL
+// 100^3 91.1 cached against 95.9 us, 110^3 125.3 against 129.1, 120^3 149.1
+// against 151.7; 9-point CRS 1500 x 1500 101.7 against 97.7).
 inline bool loop_streams(int64_t n, int64_t matrix_bytes) {
-  return (matrix_bytes + 40) * n > (int64_t(1) << 28);
+  return n > (1 << 21) && (matrix_bytes + 40) * n > (int64_t(1) << 28);
 }
 // 32-bit byte offsets address a stream.
 inline bool sym64_fits(int64_t n) { return 8 * n <= (1ll << 32); }
