@@ -90,6 +90,23 @@ def sym64_bytes(n: int, ndiag: int) -> int:
     return 8 * (1 + ndiag // 2) * n + 16 * n
 
 
+def mirrored(rows, diagonal, values, offs) -> bool:
+    """Whether the matrix with these entries (CRS order, FP64 or FP32 values;
+    diagonal = column - row, offs its distinct values, ascending) has one to
+    three mirrored pairs of diagonals and equals its transpose bit for bit."""
+    import numpy as np
+
+    upper = [o for o in offs if o > 0]
+    if not 1 <= len(upper) <= 3 or [-o for o in offs[::-1]] != list(offs):
+        return False
+    for o in upper:
+        up, lo = diagonal == o, diagonal == -o
+        if not (np.array_equal(rows[up], rows[lo] - o)
+                and values[up].tobytes() == values[lo].tobytes()):
+            return False
+    return True
+
+
 def algorithmic_bytes(short: str, meta: dict):
     """Bytes a launch must move at least (each array once, x once per SpMV)."""
     n, nnz, D = meta["n"], meta["nnz"], meta["ndiag"]
@@ -372,9 +389,16 @@ def main() -> int:
     nnz_nd = nnz - n  # the scaled operator stores no diagonal
     layout = ctx.fp32_layout()
     rows = np.repeat(np.arange(n, dtype=np.int64), np.diff(m.ptr))
-    offs = np.unique(m.index.astype(np.int64) - rows)
+    diagonal = m.index.astype(np.int64) - rows
+    offs = np.unique(diagonal)
     ndiag = int(offs.size - (offs == 0).sum())
-    del rows
+    # the FP64 products read the symmetric diagonals of such a matrix, in both formats
+    sym64 = mirrored(rows, diagonal, m.value, offs)
+    # and the FP32 product of the scaled operator, of three pairs
+    s = 1.0 / np.sqrt(m.diagonal())
+    sym32 = layout == "DIA" and ndiag == 6 and mirrored(
+        rows, diagonal, ((m.value * s[rows]) * s[m.index]).astype(np.float32), offs)
+    del rows, diagonal, s
     # operator stream of one FP32 SpMV of the scaled operator (without x, y)
     op_bytes = {"DIA": 4 * ndiag * n, "ELL": 8 * nnz_nd + 4 * n,
                 "CRS": 8 * nnz_nd + 4 * (n + 1)}[layout]
@@ -487,9 +511,7 @@ def main() -> int:
         xs[fmt] = ctx.download("X")
         prof = run64(profile=1)
         spmv_ms = per(prof, "matvec")
-        # the stencil is symmetric bit for bit: its products read the symmetric
-        # diagonals in both formats
-        by = sym64_bytes(n, ndiag) if 0 < ndiag <= 6 else \
+        by = sym64_bytes(n, ndiag) if sym64 else \
             crs_bytes(n, nnz, 8, 8) if fmt == "CRS" else ell_bytes(n, nnz, 8, 8)
         plain_ms = ctx.time_matvec("P", "Q", reps=20)
         fp64[fmt] = {
@@ -515,7 +537,9 @@ def main() -> int:
 
     secmj, infomj = timed(mixed, "mixed jacobi")
     profmj = mixed(profile=1)
-    spmv_nd_bytes = op_bytes + 8 * n  # FP32 scaled operator, x and y
+    # FP32 scaled operator (its upper diagonals only where they are all the
+    # product reads), x and y
+    spmv_nd_bytes = (op_bytes // 2 if sym32 else op_bytes) + 8 * n
     mixed_j = {
         "seconds": secmj, "iterations": infomj["iterations"],
         "reliable_updates": infomj["updates"], "true_relative_residual": infomj["true_residual"],

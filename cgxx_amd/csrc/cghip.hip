@@ -1644,8 +1644,10 @@ int cghip_mixed_iteration_bytes(const cghip_ctx *c, int precond, double *bytes) 
   // operator stream of one SpMV: FP32 values in the CG SpMV (DIA: one
   // stream per diagonal, no mask); the Clenshaw steps read DIA's FP16 row
   // records, or with symmetric storage its upper diagonals (2 bytes per
-  // stored pair; the lower values are those of earlier rows).  A product that
-  // reads the upper FP32 diagonals only (Dia::sym32) moves half of op32
+  // stored pair; the lower values are those of earlier rows).  The model
+  // prices the stored FP32 operator whole, also where the CG SpMV moves half of
+  // it (Dia::sym32: the upper diagonals only), so it is above the bytes that
+  // such an iteration moves by 2 d n
   const double op32 = c->dia_nd ? 4.0 * d * n : c->ell_nd ? 8.0 * nnz + 4.0 * n
                                                           : 8.0 * nnz + 4.0 * (n + 1);
   const double op16 = !(c->dia_nd && c->poly_fp16) ? op32

@@ -11,6 +11,7 @@ NT, ROWS, SYM.
 import importlib.util
 import os
 
+import numpy as np
 import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -51,3 +52,28 @@ def test_other_kernels_unchanged(bench):
     assert bench.algorithmic_bytes("k_mp_matvec_dot<2>", META) == 4 * 6 * n + 8 * n
     assert bench.algorithmic_bytes("k_pcg_xpay<true>", META) == 48 * n
     assert bench.algorithmic_bytes("k_unknown", META) is None
+
+
+def test_mirrored(bench):
+    """The matrices whose FP64 products read symmetric diagonals."""
+    from cgxx_amd import problems
+
+    def entries(m):
+        rows = np.repeat(np.arange(m.n, dtype=np.int64), np.diff(m.ptr))
+        diagonal = m.index.astype(np.int64) - rows
+        return rows, diagonal, m.value, np.unique(diagonal)
+
+    m = problems.diffusion3d(6, seed=3)
+    rows, diagonal, value, offs = entries(m)
+    assert bench.mirrored(rows, diagonal, value, offs)
+    assert bench.mirrored(*entries(problems.laplace2d(5)))
+    e = np.flatnonzero(diagonal > 0)[4]
+    changed = value.copy()
+    changed[e] = np.nextafter(changed[e], 0)
+    assert not bench.mirrored(rows, diagonal, changed, offs)
+    keep = np.arange(rows.size) != e
+    assert not bench.mirrored(rows[keep], diagonal[keep], value[keep], offs)
+    keep = diagonal >= 0
+    assert not bench.mirrored(rows[keep], diagonal[keep], value[keep], offs[offs >= 0])
+    keep = diagonal == 0
+    assert not bench.mirrored(rows[keep], diagonal[keep], value[keep], offs[offs == 0])
