@@ -63,9 +63,6 @@ struct cghip_ctx {
   double *pq1 = nullptr;
   size_t pq1_cap = 0;
   double *dot_out = nullptr;
-  // second buffer of P in the FP64 loop of two kernels; allocated by a solve
-  // that runs it
-  double *p_alt = nullptr;
 
   // solver
   SolveState *d_state = nullptr;
@@ -224,7 +221,7 @@ void free_fp32(cghip_ctx *c) {
 }
 
 void free_sym(Sym64 &s) {
-  if (s.diag) (void)hipFree((void *)s.diag);  // up lies in the same allocation
+  if (s.diag) (void)hipFree((void *)s.diag);  // up and p_alt lie in the same allocation
   s = Sym64{};
 }
 
@@ -331,6 +328,12 @@ const Sym64 &sym_of(const cghip_ctx *c) {
   return c->format == CGHIP_FORMAT_CRS ? c->crs_sym : c->ell_sym;
 }
 
+// The symmetric diagonals' allocation: diag, up and p_alt, each from a line on.
+size_t whole_lines(int64_t n) { return ((size_t)n + 63) / 64 * 64; }
+size_t sym_streams(const Sym64 &S) { return whole_lines(S.pairs * ((int64_t)S.n + kSym64Pad)); }
+// Second buffer of P in the FP64 loop of two kernels.
+double *p_alt_of(const Sym64 &S) { return const_cast<double *>(S.up) + sym_streams(S); }
+
 // Bytes per row that one FP64 product reads of the matrix.
 int64_t matrix_row_bytes(const cghip_ctx *c) {
   if (sym_of(c).pairs) return 8 * (1 + sym_of(c).pairs);
@@ -422,8 +425,9 @@ int find_offsets(cghip_ctx *c, const M &A, Offsets *out) {
 
 // The symmetric diagonals of an uploaded matrix, if it has them: every
 // off-diagonal offset mirrored, at most kSym64Pairs pairs, every entry equal
-// to its transpose.  Not built (no error) otherwise, or where the device has
-// no memory left for them.
+// to its transpose; and where such a system runs the loop of two kernels, its
+// second buffer of P (p_alt_of), so that a solve allocates nothing.  Not built
+// (no error) otherwise, or where the device has no memory left for them.
 template <typename M>
 int build_sym(cghip_ctx *c, const M &A, const Offsets &o, Sym64 *out) {
   const int m = o.count;
@@ -436,9 +440,9 @@ int build_sym(cghip_ctx *c, const M &A, const Offsets &o, Sym64 *out) {
   for (int k = 0; k < S.pairs; k++) S.off[k] = o.off[S.pairs + k];
   int *found = reinterpret_cast<int *>(c->partial);
   double *diag = nullptr, *up = nullptr;
-  const size_t rows = ((size_t)A.n + 63) / 64 * 64;
-  const size_t streams = (size_t)S.pairs * ((size_t)A.n + kSym64Pad);
-  if (hipMalloc((void **)&diag, sizeof(double) * (rows + streams)) != hipSuccess) {
+  const size_t rows = whole_lines(A.n);
+  const size_t p_alt = ell_chunks(A.n) <= kSmallChunks ? rows : 0;
+  if (hipMalloc((void **)&diag, sizeof(double) * (rows + sym_streams(S) + p_alt)) != hipSuccess) {
     (void)hipGetLastError();
     return CGHIP_OK;
   }
@@ -534,7 +538,6 @@ int cghip_destroy(cghip_ctx *c) {
   dfree(c->pq1);
   dfree(c->d_poly);
   dfree(c->dot_out);
-  dfree(c->p_alt);
   dfree(c->d_state);
   dfree(c->d_mstate);
   dfree(c->d_hist);
@@ -558,7 +561,6 @@ int cghip_set_size(cghip_ctx *c, int n) {
     free_fp32(c);
     free_ell(c);
     dfree(c->jac);
-    dfree(c->p_alt);
     c->has_jac = false;
     c->format = 0;
     c->n = 0;
@@ -908,11 +910,11 @@ int enqueue_first_product(cghip_ctx *c) {
 // One iteration of it: p in P before an even one, in p_alt before an odd one.
 int enqueue_two_kernels(cghip_ctx *c, const double *C, History h, bool odd) {
   double *p = c->vec[CGHIP_VEC_P], *q = c->vec[CGHIP_VEC_Q], *r = c->vec[CGHIP_VEC_R],
-         *x = c->vec[CGHIP_VEC_X];
+         *x = c->vec[CGHIP_VEC_X], *alt = p_alt_of(sym_of(c));
   const Partials pq1{c->pq1, nullptr};
   HIPCHK(c, pcg_update_small(c->n, ell_chunks(c->n), r, q, C, pq1, pr_of(c), c->d_state, h,
                              c->stream));
-  HIPCHK(c, pcg_step_sym64(sym_of(c), x, odd ? c->p_alt : p, odd ? p : c->p_alt, q, r, C, pr_of(c),
+  HIPCHK(c, pcg_step_sym64(sym_of(c), x, odd ? alt : p, odd ? p : alt, q, r, C, pr_of(c),
                            pq1, c->d_state, h, c->stream));
   return CGHIP_OK;
 }
@@ -992,11 +994,7 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
   if (o->batch <= 0) batch = std::min(batch, o->max_iter);
   if (mode == CGHIP_PROFILE_KERNELS) batch = 1;
   const bool two = mode == CGHIP_PROFILE_NONE && two_kernels(c);
-  if (two) {
-    batch += batch & 1;  // every batch starts with p in P
-    if (!c->p_alt)
-      if (int rc = dalloc(c, &c->p_alt, (size_t)c->n)) return rc;
-  }
+  if (two) batch += batch & 1;  // every batch starts with p in P
   // events[0..1] bracket the set-up; events[2..5] the kernels of an iteration.
   if (mode != CGHIP_PROFILE_NONE && ensure_events(c, 6)) return CGHIP_ERR_HIP;
   hipEvent_t *ev = mode != CGHIP_PROFILE_NONE ? c->events.data() : nullptr;
@@ -1084,7 +1082,7 @@ int cghip_solve(cghip_ctx *c, const cghip_solve_opts *o, cghip_solve_info *info)
     // p changed its buffer in every iteration but a converging one
     const Scalars &nx = c->h_state->next;
     if (two && ((nx.iteration - (nx.residual <= o->tol ? 1 : 0)) & 1)) {
-      HIPCHK(c, hipMemcpyAsync(c->vec[CGHIP_VEC_P], c->p_alt, sizeof(double) * (size_t)c->n,
+      HIPCHK(c, hipMemcpyAsync(c->vec[CGHIP_VEC_P], p_alt_of(sym_of(c)), sizeof(double) * (size_t)c->n,
                                hipMemcpyDeviceToDevice, c->stream));
       if (int rc = sync(c)) return rc;
     }

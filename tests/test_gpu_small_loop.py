@@ -118,3 +118,35 @@ def test_dot_without_allocation(ctx, n):
     assert C.CDLL("libamdhip64.so.7").hipDeviceSynchronize() == 0
     want = oracle.lib().orc_dot_tree(n, a[1:n + 1].copy(), b[1:n + 1].copy()) if n else 0.0
     assert_bitwise([ctx.download("Z")[0]], [want], "<a, b>")
+
+
+@pytest.mark.parametrize("fmt", ["CRS", "ELL"])
+def test_solve_allocates_nothing(ctx, fmt):
+    """The second buffer of P comes with the matrix: a solve of the loop of two
+    kernels leaves the device's free memory as it was (2 MB a vector), once
+    a loop of three has made the history's buffers."""
+    from tests.cases import to_ell
+
+    def free():
+        # the HIP runtime that the library itself is linked against (same soname)
+        left, total = C.c_size_t(), C.c_size_t()
+        assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(left), C.byref(total)) == 0
+        return left.value
+
+    n = 1024 * 256
+    m = banded(n, (1, 64, 4096), 23)
+    value = m[2].copy()
+    value[1] *= 1.5  # not symmetric: three kernels
+    for last in (value, m[2]):
+        ctx.set_size(n)
+        if fmt == "CRS":
+            ctx.upload_crs(m[0], m[1], last)
+        else:
+            ctx.upload_ell(*to_ell(m[0], m[1], last))
+        ctx.set_format(fmt)
+        ctx.fill("K", 1.0)
+        ctx.fill("X", 0.0)
+        before = free()
+        ctx.solve(precond="none", max_iter=9, tol=1e-300)
+        after = free()
+    assert before - after < 8 * n
