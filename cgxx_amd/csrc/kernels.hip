@@ -556,8 +556,8 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(8))) voi
   const double a = st->alpha;
   const bool converged = end_iteration(st, c, r2, rho, b, h);
   // x += a p always; p = z + b p unless the loop stops here.  Four streams
-  // per element: unrolled twice to stay within 64 VGPRs.  x, r and C are
-  // streamed non-temporally: only p stays cached for the next SpMV.
+  // per element: unrolled twice to stay within 64 VGPRs.  NT: x, r and C are
+  // streamed non-temporally, so that p stays cached for the next SpMV.
   if (converged) {
     for (int64_t g = P.q; g < P.npair; g += P.T)
       for (int64_t e = 2 * g; e < 2 * g + 2 && e < n; e++) x[e] = x[e] + a * p[e];
