@@ -90,6 +90,16 @@ def sym64_bytes(n: int, ndiag: int) -> int:
     return 8 * (1 + ndiag // 2) * n + 16 * n
 
 
+def entry_diagonals(m):
+    """Row and diagonal (column - row) of every entry, and the distinct
+    diagonals, ascending."""
+    import numpy as np
+
+    rows = np.repeat(np.arange(m.n, dtype=np.int64), np.diff(m.ptr))
+    diagonal = m.index.astype(np.int64) - rows
+    return rows, diagonal, np.unique(diagonal)
+
+
 def mirrored(rows, diagonal, values, offs) -> bool:
     """Whether the matrix with these entries (CRS order, FP64 or FP32 values;
     diagonal = column - row, offs its distinct values, ascending) has one to
@@ -388,9 +398,7 @@ def main() -> int:
     ctx.upload("K", k)
     nnz_nd = nnz - n  # the scaled operator stores no diagonal
     layout = ctx.fp32_layout()
-    rows = np.repeat(np.arange(n, dtype=np.int64), np.diff(m.ptr))
-    diagonal = m.index.astype(np.int64) - rows
-    offs = np.unique(diagonal)
+    rows, diagonal, offs = entry_diagonals(m)
     ndiag = int(offs.size - (offs == 0).sum())
     # the FP64 products read the symmetric diagonals of such a matrix, in both formats
     sym64 = mirrored(rows, diagonal, m.value, offs)
@@ -692,11 +700,11 @@ def poisson128(args) -> int:
     (N = 2,097,152, 14,581,760 nonzeros, values 6/-1), k = A*1, x0 = 0,
     Jacobi, stop at relative residual 1e-9: the fused device loop and the
     reference's loop hook by hook, in CRS and in ELL; each hook's kernel
-    time and GB/s (algorithmic bytes: SpMV as in crs_bytes/ell_bytes, dot
-    16 N, axpy/xpay/Jacobi 24 N, copy 16 N); beside them the oracle's
-    SerialCG port (1 core) and OpenMP port (up to 16 threads), full solves
-    on this host.  The matrix (217 MB) fits in the 256 MB last-level cache,
-    so the rates are effective ones.  Prints one JSON object."""
+    time and GB/s (algorithmic bytes: SpMV as in sym64_bytes, since the
+    system equals its transpose, dot 16 N, axpy/xpay/Jacobi 24 N, copy
+    16 N); beside them the oracle's SerialCG port (1 core) and OpenMP port
+    (up to 16 threads), full solves on this host.  What the loop reads (151 MB) fits in the 256 MB last-level
+    cache, so the rates are effective ones.  Prints one JSON object."""
     import numpy as np
 
     from cgxx_amd import problems
@@ -714,6 +722,8 @@ def poisson128(args) -> int:
     log(f"128^3 Poisson: N={n} nnz={nnz}")
     out = {"workload": "3D 7-point Poisson 128^3 (6/-1), k=A*1, x0=0, Jacobi, relative residual 1e-9",
            "n": n, "nnz": nnz, "formats": {}}
+    rows, diagonal, offs = entry_diagonals(m)
+    sym64 = mirrored(rows, diagonal, m.value, offs)
     vec_bytes = {"dot": 16 * n, "axpy": 24 * n, "xpay": 24 * n, "jacobi": 24 * n, "cpy": 16 * n}
     for fmt in ("CRS", "ELL"):
         ctx.set_format(fmt)
@@ -734,8 +744,8 @@ def poisson128(args) -> int:
         sec_h = time.perf_counter() - t0
         for v in ("P", "R", "Q", "Z"):
             ctx.fill(v, 1.0)
-        by = {"matvec": crs_bytes(n, nnz, 8, 8) if fmt == "CRS" else ell_bytes(n, nnz, 8, 8),
-              **vec_bytes}
+        by = {"matvec": sym64_bytes(n, offs.size - 1) if sym64 else
+              crs_bytes(n, nnz, 8, 8) if fmt == "CRS" else ell_bytes(n, nnz, 8, 8), **vec_bytes}
         hooks = {}
         for h in ("matvec", "dot", "axpy", "xpay", "jacobi", "cpy"):
             ms = ctx.time_hook(h, reps=50)

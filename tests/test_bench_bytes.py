@@ -59,9 +59,8 @@ def test_mirrored(bench):
     from cgxx_amd import problems
 
     def entries(m):
-        rows = np.repeat(np.arange(m.n, dtype=np.int64), np.diff(m.ptr))
-        diagonal = m.index.astype(np.int64) - rows
-        return rows, diagonal, m.value, np.unique(diagonal)
+        rows, diagonal, offs = bench.entry_diagonals(m)
+        return rows, diagonal, m.value, offs
 
     m = problems.diffusion3d(6, seed=3)
     rows, diagonal, value, offs = entries(m)
